@@ -43,13 +43,17 @@ typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kPfQt = 2;           // 16-row query tiles per wavefront
 constexpr int kPfWaves = 8;        // wavefronts per workgroup
 constexpr int kPfWavesPerEu = 2;
+constexpr int kPfXcds = 8;
 constexpr int kPfThreads = 64 * kPfWaves;
 constexpr int kPfRows = 16 * kPfQt * kPfWaves;  // query rows (token x head) per workgroup
 constexpr int kPfKeys = 64;        // keys per LDS tile
 constexpr int kPfDim = 128;
-// K and V tiles in LDS: key-major rows of 256 bytes whose 16-byte chunks
-// are XOR-swizzled by the row (chunk c of row r at slot c ^ (r & 15)), so
-// the fragment reads of 16 consecutive rows cover all banks.
+// K and V tiles in LDS: key-major rows of 256 bytes whose 16-byte chunks are
+// XOR-swizzled by the row (chunk c of row r at slot c ^ tile_swizzle(r)): K by
+// r % 16, so the fragment reads of 16 consecutive rows cover all banks; V by
+// 2 (r % 8), so the 32-byte pieces that 32 lanes of a transposing read take
+// from 8 consecutive rows do (swizzled like K they met two to a bank: 135 M
+// of 406 M LDS cycles at 4 x 8192 tokens, H 8, G 4, now none).
 constexpr int kKRow = 256;
 constexpr int kKBytes = kPfKeys * kKRow;   // 16384 (K or V)
 constexpr float kLazyMax = 8.f;  // log2 headroom of the softmax reference max
@@ -67,6 +71,7 @@ struct PrefillParams {
   int64_t bt_stride;
   int64_t num_pages;
   int kvh, group, num_seqs, tiles_per_seq;
+  int head_sets;  // largest of 8, 4, 2, 1 that divides kvh
   float scale_log2;
   int causal;
 };
@@ -117,25 +122,39 @@ __device__ __forceinline__ pf_rsrc_t tile_rsrc(const uint16_t* base, int64_t pag
                                            0x00020000);
 }
 
-// Loads a 64-key tile of K and of V straight into LDS (buffer_load ... lds):
-// rows of 256 bytes, 16-byte chunk c of row r at slot c ^ (r & 15).  Each
-// wave instruction fills 1 KB = four rows, lane L the slot L % 16 of row
-// L / 16, so lane L fetches chunk (L % 16) ^ (row & 15).  Rows past the
-// tile's ``nkeys`` repeat its last row: V rows stay finite (their P is 0)
-// and every load stays inside the page.
+// Transfers a 64-key tile of K and of V straight into LDS (buffer_load ...
+// lds): rows of 256 bytes, 16-byte chunk c of row r at slot c ^ swizzle(r).
+// Each wave instruction fills 1 KB = four rows, lane L the slot L % 16 of row
+// L / 16, so lane L fetches chunk (L % 16) ^ swizzle(row).  ``off`` holds the
+// lane's byte offsets in a whole tile; rows past the tile's ``nkeys`` repeat
+// its last row: V rows stay finite (their P is 0) and every load stays inside
+// the page.
+constexpr int kLoads = kPfKeys / kPfWaves / 4;  // transfer instructions per wave, tile and operand, four rows each
+template <bool kV>
+__device__ __forceinline__ int tile_swizzle(int r) {
+  return kV ? 2 * (r & 7) : r & 15;
+}
+struct TileOffsets {
+  int k[kLoads], v[kLoads];
+};
 __device__ __forceinline__ void load_tile(const PrefillParams& p, int64_t page, int key0, int nkeys, int h,
-                                          uint8_t* kst, uint8_t* vst) {
+                                          uint8_t* kst, uint8_t* vst, TileOffsets off) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = p.kvh * kPfDim * 2;  // bytes between consecutive keys
   const pf_rsrc_t rk = tile_rsrc(p.wk, page, key0, h, p.kvh);
   const pf_rsrc_t rv = tile_rsrc(p.wv, page, key0, h, p.kvh);
-  constexpr int kRows = kPfKeys / kPfWaves;  // rows per wave, four per instruction
+  if (nkeys < kPfKeys) {
 #pragma unroll
-  for (int i = 0; i < kRows / 4; ++i) {
-    const int r0 = kRows * w + 4 * i, r = r0 + (lane >> 4);
-    const int off = min(r, nkeys - 1) * row + 16 * ((lane & 15) ^ (r & 15));
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (pf_lds_ptr_t)(kst + r0 * kKRow), 16, off, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (pf_lds_ptr_t)(vst + r0 * kKRow), 16, off, 0, 0, 0);
+    for (int i = 0; i < kLoads; ++i) {
+      const int r = 4 * (kLoads * w + i) + (lane >> 4), at = min(r, nkeys - 1) * (p.kvh * kPfDim * 2);
+      off.k[i] = at + 16 * ((lane & 15) ^ tile_swizzle<false>(r));
+      off.v[i] = at + 16 * ((lane & 15) ^ tile_swizzle<true>(r));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int r0 = 4 * (kLoads * w + i);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (pf_lds_ptr_t)(kst + r0 * kKRow), 16, off.k[i], 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (pf_lds_ptr_t)(vst + r0 * kKRow), 16, off.v[i], 0, 0, 0);
   }
 }
 
@@ -160,10 +179,20 @@ __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu
   __shared__ __align__(16) uint8_t pf_k1[kKBytes];
   __shared__ __align__(16) uint8_t pf_v0[kKBytes];
   __shared__ __align__(16) uint8_t pf_v1[kKBytes];
-  const int h = blockIdx.y;
-  // longest query tiles first: later tiles see more keys under the causal mask
-  const int b = blockIdx.x % p.num_seqs;
-  const int qtile = p.tiles_per_seq - 1 - (int)(blockIdx.x / p.num_seqs);
+  // Workgroups go to the XCDs in turn.  XCD x takes the heads = x mod
+  // head_sets (equal work each), and with fewer heads than XCDs every
+  // (8 / head_sets)-th of their query tiles; a sequence's tiles follow each
+  // other, longest first (later tiles see more keys under the causal mask).
+  // Tiles of one sequence thus spread over all XCDs and CUs: with the
+  // sequence as the fastest index a long one among short ones ran on a
+  // quarter of the device (prompts of 1000, 37, 2311 and 512 tokens at H 8,
+  // G 4: 218 us, now 81 us).
+  const int xcd = (int)blockIdx.x % kPfXcds, share = kPfXcds / p.head_sets;
+  const int item = (int)blockIdx.x / kPfXcds * share + xcd / p.head_sets;
+  const int h = xcd % p.head_sets + p.head_sets * (int)blockIdx.y;
+  const int b = item / p.tiles_per_seq;
+  const int qtile = p.tiles_per_seq - 1 - item % p.tiles_per_seq;
+  if (b >= p.num_seqs) return;
   const int q0 = p.cu_q[b], qlen = p.cu_q[b + 1] - q0;
   const int T = kPfRows / p.group;  // query tokens per tile
   const int t0 = qtile * T;
@@ -222,10 +251,21 @@ __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu
     if ((pi & ~63) != pbase) {
       pbase = pi & ~63;
       pages = pbase + lane < (kend + 127) / 128 ? bt[pbase + lane] : 0;
+      // waited for here: where the paths join, the wait would also be for the
+      // transfers in flight
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     }
     return __builtin_amdgcn_readlane(pages, pi & 63);
   };
-  if (ntiles > 0) load_tile(p, page_of(0), 0, min(kPfKeys, kend), h, pf_k0, pf_v0);
+  TileOffsets offs;
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int r = 4 * (kLoads * w + i) + (lane >> 4), at = r * (p.kvh * kPfDim * 2);
+    offs.k[i] = at + 16 * ((lane & 15) ^ tile_swizzle<false>(r));
+    offs.v[i] = at + 16 * ((lane & 15) ^ tile_swizzle<true>(r));
+  }
+  if (ntiles > 0) load_tile(p, page_of(0), 0, min(kPfKeys, kend), h, pf_k0, pf_v0, offs);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
   // Nothing in flight at the loop entry (Q and the first tile have landed):
   // without this explicit wait the counter pass, merging the entry path,
@@ -235,13 +275,13 @@ __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu
   // V fragment lanes: row x = 4 q4 + j / 4 of each 16-row block, byte
   // 8 (j & 1) of the chunk; the chunk's slot term 16 ((j >> 1 & 1) ^ x)
   const int vx = 4 * q4 + (j >> 2);
-  const int vlane = vx * kKRow + 8 * (j & 1), vsw = 16 * (((j >> 1) & 1) ^ vx);
+  const int vlane = vx * kKRow + 8 * (j & 1), vsw = 16 * (((j >> 1) & 1) ^ tile_swizzle<true>(vx));
   auto tile = [&](int it, const uint8_t* stage, uint8_t* knext, const uint8_t* vstage, uint8_t* vnext)
                   __attribute__((always_inline)) {
     const int key0 = it * kPfKeys;
     const bool more = it + 1 < ntiles;
     if (more)
-      load_tile(p, page_of(key0 + kPfKeys), key0 + kPfKeys, min(kPfKeys, kend - key0 - kPfKeys), h, knext, vnext);
+      load_tile(p, page_of(key0 + kPfKeys), key0 + kPfKeys, min(kPfKeys, kend - key0 - kPfKeys), h, knext, vnext, offs);
 
     // ---- S^T = K Q^T: s[kt][qt], keys key0 + 16 kt + 4 q4 + r ----
     // The tile runs in halves so that one half's exponentials overlap the
@@ -410,6 +450,7 @@ __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu
         for (int r = 0; r < 4; ++r) psum += e[kt][qt][r];
       l[qt] += psum;
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile has landed
     __syncthreads();
   };
   for (int it = 0; it < ntiles; it += 2) {
@@ -471,11 +512,19 @@ extern "C" int fp_prefill_attention(const void* q, int64_t q_stride, const void*
   p.group = (int)group;
   p.num_seqs = (int)num_seqs;
   p.tiles_per_seq = (int)tiles;
+  p.head_sets = 1;
+  for (int sets = kPfXcds; sets > 1; sets /= 2)
+    if (kv_heads % sets == 0 && tiles * num_seqs * sets < (1LL << 31)) {
+      p.head_sets = sets;
+      break;
+    }
+  const int64_t share = kPfXcds / p.head_sets, per_xcd = (tiles * num_seqs + share - 1) / share;
   p.scale_log2 = (float)(scale * 1.4426950408889634);
   p.causal = causal ? 1 : 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // all LDS is static (two K and two V stages, 64 KB)
-  hipLaunchKernelGGL(prefill_kernel, dim3((unsigned)(tiles * num_seqs), (unsigned)kv_heads), dim3(kPfThreads), 0, s, p);
+  hipLaunchKernelGGL(prefill_kernel, dim3((unsigned)(kPfXcds * per_xcd), (unsigned)(kv_heads / p.head_sets)),
+                     dim3(kPfThreads), 0, s, p);
   FP_LAUNCH_CHECK();
   return 0;
 }

@@ -113,3 +113,9 @@ def test_long_sequence():
 
 def test_empty_sequences_in_batch():
     _run(14, heads=2, group=2, q_lens=[0, 17, 0, 130], k_lens=[0, 17, 40, 130])
+
+
+@pytest.mark.parametrize("heads,q_lens", [(3, [300, 5]), (4, [129, 64, 257]), (8, [1, 70]), (12, [260]), (16, [33, 0, 90])])
+def test_workgroup_mapping(heads, q_lens):
+    # head counts that split the XCDs 1, 4 and 8 ways; tile counts that are no multiple of the share
+    _run(50 + heads, heads=heads, group=2, q_lens=q_lens, k_lens=[n + 40 * (i % 2) for i, n in enumerate(q_lens)])
