@@ -129,11 +129,15 @@ class Extension:
             "fp_paged_set_streaming": [_i32],
             "fp_prefill_attention": [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _f64,
                                      _i32, _p, _i64, _p],
+            "fp_prefill_attention_split": [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64,
+                                           _i64, _f64, _i32, _p, _i64, _p, _i64, _p],
+            "fp_prefill_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _i64],
         }
         for name, args in sigs.items():
             fn = getattr(lib, name)
             fn.argtypes = args
             fn.restype = _i32
+        lib.fp_prefill_workspace_bytes.restype = _i64
         self._fused = lib.fp_fused_decode
         self._fused_append = lib.fp_fused_decode_append
         lib.fp_last_error.restype = ctypes.c_char_p
@@ -396,10 +400,17 @@ class Extension:
                and cu_seqlens_q.numel() == n_seqs + 1, "cu_seqlens_q int32 [B + 1], seqused_k int32 [B]")
         _check(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1
                and block_table.size(0) == n_seqs, "block_table must be int32 [B, pages] with contiguous rows")
-        self._call("fp_prefill_attention", _dev(q, "q"), q.stride(0), _dev(wk, "k"), _dev(wv, "v"), wk.size(0), kvh,
-                   group, _dev(cu_seqlens_q, "cu_seqlens_q"), _dev(seqused_k, "seqused_k"),
-                   _dev(block_table, "block_table"), block_table.stride(0), n_seqs, int(max_seqlen_q),
-                   int(max_seqlen_k), float(scale), int(bool(causal)), _dev(out, "out"), out.stride(0), _stream(q))
+        # the parts of split query tiles: from the caching allocator, so ordered
+        # with this stream's work and private to the call
+        # (contexts of up to 30 key tiles never split: no call to ask)
+        ws_bytes = 0 if max_seqlen_k <= 1920 else self._lib.fp_prefill_workspace_bytes(
+            kvh, group, n_seqs, q.size(0), int(max_seqlen_q), int(max_seqlen_k))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+        self._call("fp_prefill_attention_split", _dev(q, "q"), q.stride(0), _dev(wk, "k"), _dev(wv, "v"), wk.size(0),
+                   kvh, group, _dev(cu_seqlens_q, "cu_seqlens_q"), _dev(seqused_k, "seqused_k"),
+                   _dev(block_table, "block_table"), block_table.stride(0), n_seqs, q.size(0), int(max_seqlen_q),
+                   int(max_seqlen_k), float(scale), int(bool(causal)), _dev(out, "out"), out.stride(0),
+                   ws.data_ptr() if ws_bytes else None, ws_bytes, _stream(q))
 
 
 @functools.cache

@@ -275,6 +275,24 @@ int fp_prefill_attention(const void* q, int64_t q_stride, const void* wk, const 
                          int64_t max_seqlen_k, double scale, int causal, void* out, int64_t out_stride,
                          fp_stream_t stream);
 
+/*
+ * fp_prefill_attention with a workspace, which lets the launch split the keys
+ * of long query tiles over the device's CUs and merge the parts: few query
+ * tiles, or tiles of unequal length, then still fill the chip.  total_q (the
+ * rows of q) bounds the query tiles.  workspace: device memory of
+ * fp_prefill_workspace_bytes for the same sizes, 16-byte aligned, contents
+ * irrelevant before and after; calls that may overlap need one each.  A null
+ * workspace (or 0 bytes asked for) runs fp_prefill_attention's launch.
+ */
+int fp_prefill_attention_split(const void* q, int64_t q_stride, const void* wk, const void* wv, int64_t num_pages,
+                               int64_t kv_heads, int64_t group, const int32_t* cu_seqlens_q, const int32_t* seqused_k,
+                               const int32_t* block_table, int64_t bt_stride, int64_t num_seqs, int64_t total_q,
+                               int64_t max_seqlen_q, int64_t max_seqlen_k, double scale, int causal, void* out,
+                               int64_t out_stride, void* workspace, int64_t workspace_bytes, fp_stream_t stream);
+/* Workspace bytes of fp_prefill_attention_split (0: none is used). */
+int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
+                                   int64_t max_seqlen_q, int64_t max_seqlen_k);
+
 #ifdef __cplusplus
 }
 #endif

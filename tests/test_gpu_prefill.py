@@ -119,3 +119,95 @@ def test_empty_sequences_in_batch():
 def test_workgroup_mapping(heads, q_lens):
     # head counts that split the XCDs 1, 4 and 8 ways; tile counts that are no multiple of the share
     _run(50 + heads, heads=heads, group=2, q_lens=q_lens, k_lens=[n + 40 * (i % 2) for i, n in enumerate(q_lens)])
+
+
+# Grids with fewer query tiles than CUs split their keys over the CUs
+# (fp_prefill_attention_split): P rounds as in the unsplit launch and only the
+# order of fp32 sums differs, so a BF16 output moves by at most one step
+# (2^-7 of its value), plus the sums' own rounding where terms cancel
+# (2^-24 x ~100 terms' growth, of the largest |V| ~ 5: < 1e-4).
+SPLITS = [
+    # heads, group, q lengths, key lengths, causal
+    (4, 8, [200], [8392], True),  # a short last chunk: each query tile in many parts
+    (1, 1, [1], [1600], True),  # one row, one head
+    (3, 2, [129, 0, 128, 1], [1700, 0, 3000, 1537], True),  # odd heads, an empty sequence, tile edges
+    (8, 4, [700], [2000], True),  # ranges that end one tile and start the next
+    (2, 4, [65, 64, 63], [1601, 1600, 1599], False),  # full attention
+    (1, 8, [33] * 9, [1536 + 31 * i for i in range(9)], True),  # several sequences, 32-token tiles
+    (2, 1, [256, 257], [1000, 1800], True),
+    (1, 4, [70], [64], True),  # fewer keys than queries: rows without keys
+]
+
+
+@pytest.mark.parametrize("heads,group,q_lens,k_lens,causal", SPLITS)
+def test_split_matches_unsplit(heads, group, q_lens, k_lens, causal):
+    import torch
+
+    from fragpack_amd.ops.fragpack_ext import extension
+
+    lib = extension()._lib
+    # (a key bound that makes the split's rule hold also for short keys)
+    max_q, max_k = max(q_lens), max(max(k_lens), 8192)
+    q, wk, wv, bt, cu, kl = (torch.from_numpy(x) if isinstance(x, np.ndarray) else x
+                             for x in _case(31 + len(q_lens), heads, group, q_lens, k_lens))
+    # rows concentrated on a late key: the softmax reference moves in mid-sequence
+    for b in range(len(k_lens)):
+        if k_lens[b] > 1000:
+            j = k_lens[b] * 2 // 3
+            wk[int(bt[b, j // T]), j % T] *= 12
+    width = -(-max_k // T)
+    bt = torch.nn.functional.pad(bt, (0, max(0, width - bt.shape[1])))
+    q, wk, wv, bt, cu, kl = (x.cuda() for x in (q, wk, wv, bt, cu, kl))
+    need = lib.fp_prefill_workspace_bytes(heads, group, len(q_lens), q.shape[0], max_q, max_k)
+    assert need > 0
+    ws = torch.randint(0, 255, (need,), dtype=torch.uint8, device="cuda")
+    outs = []
+    for split in (False, True):
+        print("split prefill", heads, group, q_lens, k_lens, causal, split, flush=True)
+        out = torch.full_like(q, float("nan"))
+        args = (q.data_ptr(), q.stride(0), wk.data_ptr(), wv.data_ptr(), wk.shape[0], heads, group, cu.data_ptr(),
+                kl.data_ptr(), bt.data_ptr(), bt.stride(0), len(q_lens))
+        tail = (max_q, max_k, D ** -0.5, int(causal), out.data_ptr(), out.stride(0))
+        stream = torch.cuda.current_stream().cuda_stream
+        if split:
+            rc = lib.fp_prefill_attention_split(*args, q.shape[0], *tail, ws.data_ptr(), need, stream)
+        else:
+            rc = lib.fp_prefill_attention(*args, *tail, stream)
+        assert rc == 0, lib.fp_last_error()
+        torch.cuda.synchronize()
+        outs.append(out.float())
+    assert torch.isfinite(outs[0]).all()
+    torch.testing.assert_close(outs[1], outs[0], atol=1e-4, rtol=2 ** -7)
+    if max(k_lens) > 64:
+        ref = _reference(q.cpu(), wk.cpu(), wv.cpu(), bt.cpu().numpy(), cu.cpu().numpy(), kl.cpu().numpy(), group,
+                         D ** -0.5, causal)
+        torch.testing.assert_close(outs[1].cpu(), ref, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("heads,group,q_lens,k_lens", [
+    (2, 1, [100, 300], [100, 500]),  # shares of a query tile are token ranges
+    (3, 2, [129, 1, 128], [300, 70, 128]),
+    (2, 8, [70, 33], [70, 200]),  # shares are head ranges
+])
+def test_four_and_eight_wave_workgroups_agree(heads, group, q_lens, k_lens):
+    # an inflated query bound makes the grid large: the 8-wave launch (dead
+    # tiles leave at once); the same rows per wave, so the same bits
+    import torch
+
+    from fragpack_amd.ops.prefill_attn import flash_attn_varlen_func
+
+    q, wk, wv, bt, cu, kl = _case(71 + group, heads, group, q_lens, k_lens)
+    outs = []
+    for max_q in (max(q_lens) + len(q_lens) * 256, 128 * 256):
+        print("prefill waves", heads, group, q_lens, max_q, flush=True)
+        out = torch.full_like(q, float("nan"), device="cuda")
+        # (one call over more tokens than there are: the rows bound the tiles too)
+        big = torch.zeros((max_q, heads * group, D), dtype=torch.bfloat16, device="cuda")
+        big[: q.shape[0]] = q.cuda()
+        dst = torch.empty_like(big)
+        flash_attn_varlen_func(q=big, k=wk.cuda(), v=wv.cuda(), out=dst, cu_seqlens_q=torch.from_numpy(cu).cuda(),
+                               max_seqlen_q=max_q, seqused_k=torch.from_numpy(kl).cuda(), max_seqlen_k=max(k_lens),
+                               softmax_scale=D ** -0.5, causal=True, block_table=torch.from_numpy(bt).cuda())
+        out.copy_(dst[: q.shape[0]])
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
