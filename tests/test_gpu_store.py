@@ -695,3 +695,34 @@ def test_stream_probe_copies_the_written_prefix(read_bytes, write_bytes, wg):
     assert bool((d[:, write_bytes:] == 0xA5).all())
     with pytest.raises(RuntimeError, match="write <= read"):
         extension().stream_probe(src, dst, 4096, 8192, wg)
+
+
+@pytest.mark.parametrize("heads,fits", [(2, 1), (8, 5), (16, 31)])
+def test_contended_pages_spill_only_what_does_not_fit(heads, fits):
+    """All of a block's records claim their page at once.  A page of about
+    ``fits`` records takes records until none of the spilled ones fits in what
+    is left, the records lie disjoint, and each spilled one has its own slot."""
+    page = (fits * (DENSE + 512) + 15) // 16 * 16
+    eng = SimEngine(91 + heads, layers=1, heads=heads, blocks=6, page=page, staging=2, overflow=6 * 2 * heads)
+    eng.step([("a", 6 * T)])
+    blocks = list(range(6))
+    fallbacks, spills = eng.check_records(blocks)  # bytes, disjoint places
+    fill = eng.store.fill.cpu().numpy()[0]
+    pool0, pool = eng.store.overflow.data_ptr(), eng.store.overflow.numel()
+    addr = eng.store.rec_addr.cpu().numpy()[0]
+    placed = 0
+    for b in blocks:
+        used = 0
+        for k in range(2):
+            for h in range(heads):
+                need = len(oracle.encode_record(eng.kv[0, k, b, :, h], eng.table[0, k, h], k))
+                if pool0 <= int(addr[b, k, h]) < pool0 + pool:
+                    assert need == RAW or fill[b] + need > page, "a spilled record still fits"
+                else:
+                    used += need
+                    placed += 1
+        assert fill[b] == used <= page
+    assert placed + spills + fallbacks == 6 * 2 * heads and spills > 0
+    slots = [int(a) for a in addr.reshape(-1) if pool0 <= int(a) < pool0 + pool]
+    assert len(set(slots)) == len(slots)
+    eng.check_gather()
