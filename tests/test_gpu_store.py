@@ -726,3 +726,45 @@ def test_contended_pages_spill_only_what_does_not_fit(heads, fits):
     slots = [int(a) for a in addr.reshape(-1) if pool0 <= int(a) < pool0 + pool]
     assert len(set(slots)) == len(slots)
     eng.check_gather()
+
+
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 1100])
+def test_prepare_of_many_single_tokens(n):
+    """Around one offset-0 token per thread of prepare's workgroup (its path
+    for small steps up to there): more claims than free slots, so heirs'
+    scratch and staging errors too; then closes that release and hand over
+    slots, and slots of finished requests."""
+    eng = SimEngine(7 + n, layers=1, heads=1, blocks=2 * n + 8, staging=n - 300, overflow=8, max_tokens=2 * n)
+    names = [str(i) for i in range(n)]
+    eng.step([(x, 1) for x in names])
+    for x in names[:200]:
+        eng.finish(x)
+    eng.step([(x, 1) for x in names[200:]] + [("n%d" % i, 1) for i in range(150)])
+    eng.step([("n%d" % i, 1) for i in range(150)] + [("m%d" % i, 1) for i in range(40)], pad=3)
+
+
+def test_prepare_of_a_step_with_more_closes_than_threads():
+    n = 1030
+    eng = SimEngine(5, layers=1, heads=1, blocks=n + 40, staging=4, overflow=8, max_tokens=(n + 2) * T)
+    eng.step([("a", 17)])
+    eng.step([("a", T), ("b", n * T - 5)])
+    eng.step([("a", 1), ("b", 5)])
+
+
+@pytest.mark.parametrize("n_blocks", [63, 64, 67])
+def test_prepare_with_many_table_entries(n_blocks):
+    """Around the table entries from which prepare takes a second launch
+    (64 blocks x 128 entries): every claimed record points at its staging."""
+    import torch
+
+    eng = SimEngine(3, layers=4, heads=16, blocks=80, staging=3, overflow=8, max_tokens=80 * T)
+    slots = np.concatenate([b * T + np.arange(T) for b in range(n_blocks)] + [np.arange(5) + 75 * T])
+    dev = torch.from_numpy(slots.astype(np.int64)).cuda()
+    for live in ([], [75]):  # twice: the second finds slots in use
+        eng.store.prepare(dev, dev.numel(), np.array(live, np.int32))
+        eng.model.prepare(slots.tolist(), live)
+        eng.check_bookkeeping(claims=True)
+        assert (eng.store.fill[:, :n_blocks] == 0).all()
+        eng.store.commit()
+        eng.model.commit()
+        eng.check_bookkeeping(claims=False)
