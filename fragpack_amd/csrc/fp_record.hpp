@@ -43,8 +43,8 @@ constexpr int kMaxWarpRaw = 32;
 constexpr int kRawNibble = 15;
 // Largest escape count of a coded record (VAR_CAP bounds the nibble bytes).
 constexpr int kMaxEscapes = 2 * (kVarCap - kHeaderBytes);  // 4000
-// Per-wave LDS bytes for one slab's expanded escape bytes (window reads may
-// run up to 12 bytes past the last escape, and the region starts 8-aligned).
+// LDS bytes of a record's expanded escape bytes (window reads may run up to 12
+// bytes past the last escape).
 constexpr int kEscLds = kMaxEscapes + 64;
 
 // ---------------------------------------------------------------------------
@@ -324,56 +324,6 @@ __device__ __forceinline__ uint2 expand_nibbles(uint32_t n, const uint32_t (&sl)
   const uint32_t ev = lut16(n & 0x0F0F0F0Fu, sl[0], sl[1], sl[2], sl[3]);
   const uint32_t od = lut16((n >> 4) & 0x0F0F0F0Fu, sl[0], sl[1], sl[2], sl[3]);
   return make_uint2(perm(od, ev, 0x05010400u), perm(od, ev, 0x07030602u));
-}
-
-// Record header fields one slab needs.
-struct SlabHdr {
-  int e0, e1;       // escape ordinals [e0, e1) of the slab's threads
-  int r0, r1;       // raw-list entries [r0, r1)
-  int raw_offset;   // byte offset of the raw list in the variable region
-};
-
-// ``rd4(offset)`` reads the u32 at byte ``offset`` of the variable region
-// (global memory or an LDS copy).
-// Slab ``slab`` (threads 64 slab .. 64 slab + 63) spans the header's
-// 2048-scalar prefix entries 2 slab and 2 slab + 1; the low u16 of dword
-// 4 + slab (8 + slab) is esc_prefix[2 slab] (raw_prefix[2 slab]).
-template <typename Rd4>
-__device__ __forceinline__ SlabHdr slab_header(Rd4&& rd4, int slab) {
-  SlabHdr h;
-  h.e0 = (int)(rd4(16 + 4 * slab) & 0xFFFF);
-  h.r0 = (int)(rd4(32 + 4 * slab) & 0xFFFF);
-  if (slab < 3) {
-    h.e1 = (int)(rd4(16 + 4 * (slab + 1)) & 0xFFFF);
-    h.r1 = (int)(rd4(32 + 4 * (slab + 1)) & 0xFFFF);
-  } else {
-    h.e1 = (int)rd4(0);
-    h.r1 = (int)rd4(4);
-  }
-  h.raw_offset = (int)rd4(8);
-  return h;
-}
-
-// Expands the slab's escape nibbles through the extended table into ``esc``
-// (wave-private LDS, kEscLds bytes) and patches raw scalars' high bytes from
-// the raw list.  Byte k of ``esc`` is escape ordinal (e0 & ~7) + k.  All 64
-// lanes of the wave must call this together.
-template <typename Rd4>
-__device__ __forceinline__ void stage_escapes(Rd4&& rd4, const SlabHdr& h, const uint32_t (&sl)[4], uint8_t* esc,
-                                              int lane) {
-  const int d0 = h.e0 >> 3;
-  const int nd = min(((h.e1 + 7) >> 3) - d0, kMaxEscapes / 8 + 1);
-  for (int k = lane; k < nd; k += 64) {
-    const uint2 b = expand_nibbles(rd4(kHeaderBytes + 4 * (d0 + k)), sl);
-    *reinterpret_cast<uint2*>(esc + 8 * k) = b;
-  }
-  wave_lds_sync();
-  for (int k = h.r0 + lane; k < h.r1; k += 64) {
-    const uint32_t e = rd4(h.raw_offset + 4 * k);
-    const int x = (int)(e & 0xFFFFu) - 8 * d0;
-    if (x >= 0 && x < kEscLds) esc[x] = (uint8_t)(e >> 16);
-  }
-  wave_lds_sync();
 }
 
 // Decodes the 64 scalars of one kernel-order thread of a coded record and

@@ -1479,9 +1479,15 @@ __global__ void __launch_bounds__(kPrepThreads) commit_kernel(Store s) {
 // then the tile is stored with 16-byte coalesced writes.
 
 constexpr int kTileRow = 256;  // bytes per token row in the tile
+// (36.9 KB: four workgroups per CU; with an escape area per wave it was 49 KB
+// and three, and a 64-block H 8 gather's 1024 workgroups took two rounds.
+// With that, and the variable region in flight beside the dense part instead
+// of read header first, 64 blocks take 11.6 us, 15.6 before; 256 blocks 47.6,
+// 50.7 before: 4.8 TB/s read and written, what a copy reaches.)
 struct DecShared {
   uint8_t tile[kTokens * kTileRow];
-  uint8_t esc[4][kEscLds];
+  uint8_t esc[kEscLds];  // the record's expanded escape bytes, by ordinal
+  uint32_t hdr[kHeaderBytes / 4];
 };
 
 __device__ __forceinline__ int tile_off(int tok, int dim) {
@@ -1491,7 +1497,7 @@ __device__ __forceinline__ int tile_off(int tok, int dim) {
 }
 
 __device__ void decode_record_to_tile(const uint8_t* rec, int vlen, int kv, const HeadLut& lut, DecShared& sh) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, wave = tid >> 6;
   const int w = tid >> 5, g = (tid >> 2) & 7, c = tid & 3;
   auto put = [&](int st, const uint4& wd) {
     const uint32_t d[4] = {wd.x, wd.y, wd.z, wd.w};
@@ -1510,18 +1516,39 @@ __device__ void decode_record_to_tile(const uint8_t* rec, int vlen, int kv, cons
   auto emit = [&](auto st, const uint4& wd) { put(decltype(st)::value, wd); };
   SlabBuf b;
   const bool raw = vlen > kVarCap;
+  // the thread's 8 bytes of the variable region go out with its dense loads
+  const int o = 8 * tid;
+  uint2 v = make_uint2(0u, 0u);
+  if (!raw && o < vlen) v = ld8_nt(rec + kDenseBytes + o);
   load_thread(rec, raw, tid, b);
   if (raw) {
     raw_words(b, rec, tid, emit);
     return;
   }
-  const uint8_t* var = rec + kDenseBytes;
-  auto rd4 = [&](int off) { return ld4(var + off); };
-  const SlabHdr h = slab_header(rd4, wave);
-  stage_escapes(rd4, h, lut.s, sh.esc[wave], lane);
+  // escape nibbles -> table bytes, each thread from its piece; then raw-list
+  // entries patch theirs
+  if (o < kHeaderBytes) {
+    sh.hdr[o >> 2] = v.x;
+    sh.hdr[(o >> 2) + 1] = v.y;
+  } else if (o < vlen) {
+    const uint2 e0 = expand_nibbles(v.x, lut.s), e1 = expand_nibbles(v.y, lut.s);
+    *reinterpret_cast<uint4*>(sh.esc + 2 * (o - kHeaderBytes)) = make_uint4(e0.x, e0.y, e1.x, e1.y);
+  }
+  lds_barrier();
+  const int n_raw = (int)sh.hdr[1], raw_offset = (int)sh.hdr[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int off = o + 4 * q;
+    if (off >= raw_offset && ((off - raw_offset) >> 2) < n_raw) {
+      const uint32_t e = q ? v.y : v.x;
+      const int x = (int)(e & 0xFFFFu);
+      if (x < kEscLds) sh.esc[x] = (uint8_t)(e >> 16);
+    }
+  }
+  lds_barrier();
   const int cnt = thread_escapes(b);
-  const int incl = wave_incl_scan(cnt);
-  decode_words(b, sh.esc[wave], (h.e0 & 7) + incl - cnt, lut.p0, lut.p1, emit);
+  const int first = (int)(sh.hdr[4 + wave] & 0xFFFFu);  // escapes before the wave's slab
+  decode_words(b, sh.esc, first + wave_incl_scan(cnt) - cnt, lut.p0, lut.p1, emit);
 }
 
 // Stores the tile: token row r to out + r * row_stride (bytes).
