@@ -925,9 +925,12 @@ namespace {
 // - 8-wave workgroups, one per 256-row query tile and KV head, each of whose
 //   key tiles takes ~1.7 us;
 // - 4-wave workgroups, two per query tile (its rows by halves, ~1.3 us a key
-//   tile when a CU has one), while there are no more query tiles than CUs:
-//   1024 new tokens over 2048 take 76 instead of 95 us; 4 x 1024 over 8192
-//   (512 tiles), 6% slower;
+//   tile when a CU has one), while the 8-wave ones would leave CUs idle (1024
+//   new tokens over 2048: 76 instead of 95 us), and for fresh prompts of up to
+//   four query tiles per CU, whose tiles differ in length (2311 tokens 68 us
+//   instead of 81, 4 x 1000 59 instead of 69, 2048 x 2 89 instead of 93).  On
+//   full grids of equal tiles they lose, each K / V tile serving half the rows
+//   (4 x 1024 over 8192: 598 us, 8 waves 583; 4 x 8192: 2%);
 // - the split launch: ~45 us of its own (three kernels, the parts written and
 //   read) plus ~2.3 us per key tile of a CU's share, where that beats the
 //   longest query tile by 10%: 200 new tokens over 8192 at H 4, G 8 take 82 us
@@ -950,7 +953,8 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   const int64_t most = r.tiles * num_seqs;
   const int64_t all = (total_q > 0 ? std::min(most, total_q / T + num_seqs) : most) * kv_heads;
   r.steps = all * steps;
-  r.waves = all <= cus ? 4 : kPfWaves;
+  const bool fresh = 2 * max_seqlen_k <= 3 * max_seqlen_q;
+  r.waves = 4 * all <= 3 * cus || (fresh && all <= 4 * cus) ? 4 : kPfWaves;
   // in units of 0.1 us
   const bool split = all <= cus && 10 * (450 * cus + 23 * r.steps) < 9 * cus * (100 + 13 * steps);
   r.split_wgs = total_q > 0 && split && r.steps <= kPfSplitMost ? (int)cus : 0;

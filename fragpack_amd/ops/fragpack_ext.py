@@ -383,34 +383,40 @@ class Extension:
     # -- prefill (the FlashAttention call of backend.py:560-575) --
     def prefill_attention(self, q, wk, wv, out, cu_seqlens_q, seqused_k, block_table, max_seqlen_q: int,
                           max_seqlen_k: int, scale: float, causal: bool) -> None:
+        # one tuple read per tensor property: short calls are bound by the host
+        qsh, qst, osh, ost, ksh = q.shape, q.stride(), out.shape, out.stride(), wk.shape
+        bsh, bst, bf16, i32 = block_table.shape, block_table.stride(), torch.bfloat16, torch.int32
         n_seqs = seqused_k.numel()
-        if n_seqs == 0 or q.size(0) == 0:
+        if n_seqs == 0 or qsh[0] == 0:
             return
-        _check(q.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and wk.dtype == torch.bfloat16
-               and wv.dtype == torch.bfloat16, "q / k / v / out must be BF16")
-        _check(q.dim() == 3 and q.size(2) == 128 and q.stride(2) == 1 and q.stride(1) == 128,
+        _check(q.dtype == bf16 and out.dtype == bf16 and wk.dtype == bf16 and wv.dtype == bf16,
+               "q / k / v / out must be BF16")
+        _check(len(qsh) == 3 and qsh[2] == 128 and qst[2] == 1 and qst[1] == 128,
                "q must be [N, Hq, 128] with contiguous heads")
-        _check(out.shape == q.shape and out.stride(2) == 1 and out.stride(1) == 128, "out must match q")
-        _check(wk.dim() == 4 and wk.size(1) == 128 and wk.size(3) == 128 and wk.is_contiguous()
-               and wv.shape == wk.shape and wv.is_contiguous(), "k / v must be contiguous [P, 128, H, 128]")
-        kvh = wk.size(2)
-        group = q.size(1) // kvh
-        _check(group * kvh == q.size(1), "query heads must be a multiple of the KV heads")
-        _check(cu_seqlens_q.dtype == torch.int32 and seqused_k.dtype == torch.int32
+        _check(osh == qsh and ost[2] == 1 and ost[1] == 128, "out must match q")
+        _check(len(ksh) == 4 and ksh[1] == 128 and ksh[3] == 128 and wk.is_contiguous()
+               and wv.shape == ksh and wv.is_contiguous(), "k / v must be contiguous [P, 128, H, 128]")
+        kvh = ksh[2]
+        group = qsh[1] // kvh
+        _check(group * kvh == qsh[1], "query heads must be a multiple of the KV heads")
+        _check(cu_seqlens_q.dtype == i32 and seqused_k.dtype == i32
                and cu_seqlens_q.numel() == n_seqs + 1, "cu_seqlens_q int32 [B + 1], seqused_k int32 [B]")
-        _check(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1
-               and block_table.size(0) == n_seqs, "block_table must be int32 [B, pages] with contiguous rows")
-        # the parts of split query tiles: from the caching allocator, so ordered
-        # with this stream's work and private to the call
-        # (contexts of up to 30 key tiles never split: no call to ask)
-        ws_bytes = 0 if max_seqlen_k <= 1920 else self._lib.fp_prefill_workspace_bytes(
-            kvh, group, n_seqs, q.size(0), int(max_seqlen_q), int(max_seqlen_k))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
-        self._call("fp_prefill_attention_split", _dev(q, "q"), q.stride(0), _dev(wk, "k"), _dev(wv, "v"), wk.size(0),
-                   kvh, group, _dev(cu_seqlens_q, "cu_seqlens_q"), _dev(seqused_k, "seqused_k"),
-                   _dev(block_table, "block_table"), block_table.stride(0), n_seqs, q.size(0), int(max_seqlen_q),
-                   int(max_seqlen_k), float(scale), int(bool(causal)), _dev(out, "out"), out.stride(0),
-                   ws.data_ptr() if ws_bytes else None, ws_bytes, _stream(q))
+        _check(block_table.dtype == i32 and len(bsh) == 2 and bst[1] == 1
+               and bsh[0] == n_seqs, "block_table must be int32 [B, pages] with contiguous rows")
+        # Workspace for the parts of split query tiles: from the caching
+        # allocator, so ordered with this stream's work and private to the call
+        # (contexts of up to 30 key tiles never split: no need to ask).
+        n, max_q, max_k = qsh[0], int(max_seqlen_q), int(max_seqlen_k)
+        ws, ws_bytes = None, 0
+        if max_k > 1920:
+            ws_bytes = self._lib.fp_prefill_workspace_bytes(kvh, group, n_seqs, n, max_q, max_k)
+            if ws_bytes:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+        self._call("fp_prefill_attention_split", _dev(q, "q"), qst[0], _dev(wk, "k"), _dev(wv, "v"), ksh[0], kvh,
+                   group, _dev(cu_seqlens_q, "cu_seqlens_q"), _dev(seqused_k, "seqused_k"),
+                   _dev(block_table, "block_table"), bst[0], n_seqs, n, max_q, max_k, float(scale),
+                   int(bool(causal)), _dev(out, "out"), ost[0], ws.data_ptr() if ws_bytes else None, ws_bytes,
+                   _stream(q))
 
 
 @functools.cache
