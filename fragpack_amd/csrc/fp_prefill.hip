@@ -224,7 +224,7 @@ __device__ __forceinline__ uint2 lds_tr16(const uint8_t* a) {
 // reached at its first key tile, so P rounds to the same BF16 values however
 // the work is cut, and only the fp32 sums' order differs.  The reference
 // moves only at key tiles where some column outgrows it by 2^kLazyMax; it
-// never falls, so such a tile's maximum outgrows the first tile's too.
+// never falls, so such a tile's maximum outgrows a lower bound of it too.
 // prefill_max_kernel scores every range (Q K^T only) and keeps the column
 // maxima of the tiles that do (few); a part replays them.
 constexpr int kPfMinSteps = 4;  // key tiles of a range, at least
@@ -729,7 +729,11 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 
 // Column maxima for the parts' references (see above): every range but the
 // parts that end their query tile, which none follows.  Grid as the split
-// prefill's.
+// prefill's.  Bound by its steps' latency (K fragments from LDS, one barrier a
+// key tile: ~1.1 us, 1.4 with every tile masked and its columns reduced), 25
+// us of the 76 that 200 tokens over 8192 take (H 4, G 8; 9 parts a tile); the
+// parts take 54 (14 of launch and first loads, ~7 of replays, 4 of stores,
+// ~1.9 a key tile) and the merge 10.
 __global__ void __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(kPfWavesPerEu))) prefill_max_kernel(PrefillParams p) {
   // four stages: a step is shorter than a memory round trip, so transfers run
   // three key tiles ahead
@@ -775,9 +779,18 @@ __global__ void __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per
     kmax[qt] = p.causal ? min(klen, tok + shift + 1) : klen;
   }
   const TileOffsets<kPfWaves> offs = tile_offsets<kPfWaves>(p);
-  float m0[kPfQt];
+  // A lower bound of each column's reference: key tile 0's maximum, and the
+  // later maxima less the headroom (a reference that much below would have
+  // moved).  Only a tile that outgrows it can move the reference.  (The
+  // headroom a little too wide: rounding must not lift the bound.)
+  const float lazy = kLazyMax / p.scale_log2 * 1.0001f;
+  float low[kPfQt];
 #pragma unroll
-  for (int qt = 0; qt < kPfQt; ++qt) m0[qt] = -INFINITY;
+  for (int qt = 0; qt < kPfQt; ++qt) low[qt] = -INFINITY;
+  int kmin = min(kmax[0], kmax[1]);  // wave-uniform: tiles ending past this key reach some column's limit
+#pragma unroll
+  for (int o = 32; o; o >>= 1) kmin = min(kmin, __shfl_xor(kmin, o, 64));
+  kmin = uniform(kmin);
   // key tile 0 first (its maxima are the first reference), then the range's;
   // step i works on key tile tile_of(i)
   const int n = it1 - it0 + (it0 > 0);
@@ -809,36 +822,46 @@ __global__ void __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per
     __syncthreads();                     // in every wave; and the last step's reads are done
     load(i + 3, next);
     const int it = tile_of(i), key0 = it * kPfKeys;
-    float mx[kPfQt];
-#pragma unroll
-    for (int qt = 0; qt < kPfQt; ++qt) mx[qt] = -INFINITY;
+    pf_f32x4 sc[4][kPfQt];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      pf_f32x4 s[kPfQt];
 #pragma unroll
-      for (int qt = 0; qt < kPfQt; ++qt) s[qt] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int qt = 0; qt < kPfQt; ++qt) sc[kt][qt] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const uint4 kf = *reinterpret_cast<const uint4*>(st + (16 * kt + j) * kKRow + 16 * ((4 * ks + q4) ^ tile_swizzle<false>(j)));
 #pragma unroll
-        for (int qt = 0; qt < kPfQt; ++qt) s[qt] = pf_mfma(kf, qf[qt][ks], s[qt]);
+        for (int qt = 0; qt < kPfQt; ++qt) sc[kt][qt] = pf_mfma(kf, qf[qt][ks], sc[kt][qt]);
       }
-#pragma unroll
-      for (int qt = 0; qt < kPfQt; ++qt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          mx[qt] = fmaxf(mx[qt], key0 + 16 * kt + 4 * q4 + r < kmax[qt] ? s[qt][r] : -INFINITY);
     }
+    if (key0 + kPfKeys > kmin) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int qt = 0; qt < kPfQt; ++qt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (key0 + 16 * kt + 4 * q4 + r >= kmax[qt]) sc[kt][qt][r] = -INFINITY;
+    }
+    // the lane's own maxima decide; the columns' are formed where they are kept
+    float mx[kPfQt];
     bool grow = false;
 #pragma unroll
     for (int qt = 0; qt < kPfQt; ++qt) {
-      mx[qt] = pf_xor32_max(pf_xor16_max(mx[qt]));
-      grow |= outgrows(mx[qt], m0[qt], p.scale_log2);
+      mx[qt] = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx[qt] = fmaxf(mx[qt], sc[kt][qt][r]);
+      grow |= outgrows(mx[qt], low[qt], p.scale_log2);
     }
     const bool keep = __ballot(grow) != 0;
-    if (i == 0) {
+    if (keep) {
 #pragma unroll
-      for (int qt = 0; qt < kPfQt; ++qt) m0[qt] = mx[qt];
+      for (int qt = 0; qt < kPfQt; ++qt) {
+        mx[qt] = pf_xor32_max(pf_xor16_max(mx[qt]));
+        low[qt] = fmaxf(low[qt], i == 0 ? mx[qt] : mx[qt] - lazy);
+      }
     }
     if (it < it0) return;
     const int k = it - it0;
@@ -933,7 +956,7 @@ namespace {
 //   (4 x 1024 over 8192: 598 us, 8 waves 583; 4 x 8192: 2%);
 // - the split launch: ~45 us of its own (three kernels, the parts written and
 //   read) plus ~2.3 us per key tile of a CU's share, where that beats the
-//   longest query tile by 10%: 200 new tokens over 8192 at H 4, G 8 take 82 us
+//   longest query tile by 10%: 200 new tokens over 8192 at H 4, G 8 take 76 us
 //   instead of 175 (4 waves) or 226 (8).
 constexpr int64_t kPfSplitMost = 1 << 16;  // key tiles (1 KB of workspace each)
 
