@@ -74,7 +74,9 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-def _store_desc(state: tuple[torch.Tensor, ...]) -> FpStore:
+def store_desc(state: tuple[torch.Tensor, ...]) -> FpStore:
+    """The C descriptor of a store's 13 state tensors (checked).  It holds
+    their addresses: the caller keeps the tensors."""
     (counters, wslot, tags, free_stack, ovf_bits, claim_list, close_list, rec_addr, rec_len, staging, scratch,
      overflow, fill) = state
     _check(rec_addr.dim() == 4 and rec_addr.dtype == torch.int64, "rec_addr must be int64 [L, NB, 2, H]")
@@ -207,15 +209,17 @@ class Extension:
             plan._fp_plan_key = (units, B, kvh)
 
     # -- store (fragpack_ext.cpp:11-39, hbm_kv.cu:669-734) --
-    def hbm_prepare(self, *args) -> None:
+    # ``desc``: the state's store_desc, for a caller that owns the 13 tensors
+    # and made it once (building it reads every tensor's properties).
+    def hbm_prepare(self, *args, desc: FpStore | None = None) -> None:
         state, (slot_mapping, n_tok, live, n_live, step) = args[:13], args[13:]
         _check(slot_mapping.dtype == torch.int64, "slot_mapping must be int64")
-        d = _store_desc(state)
+        d = store_desc(state) if desc is None else desc
         _check(2 * int(n_tok) <= state[5].numel(), "block lists too small")
         self._call("fp_hbm_prepare", ctypes.byref(d), _dev(slot_mapping, "slot_mapping"), int(n_tok),
                    _dev(live, "live"), int(n_live), int(step), _stream(slot_mapping))
 
-    def hbm_write(self, *args) -> None:
+    def hbm_write(self, *args, desc: FpStore | None = None) -> None:
         state, (key, value, slot_mapping, layer) = args[:13], args[13:]
         n = key.size(0)
         if n == 0:
@@ -223,41 +227,41 @@ class Extension:
         _check(key.stride(2) == 1 and value.stride(2) == 1, "head dim must be contiguous")
         _check(key.dtype == torch.bfloat16 and value.dtype == torch.bfloat16, "K / V must be BF16")
         _check(slot_mapping.dtype == torch.int64 and slot_mapping.numel() >= n, "slot_mapping must be int64 [N]")
-        d = _store_desc(state)
+        d = store_desc(state) if desc is None else desc
         _check(key.size(1) == d.kv_heads and key.size(2) == 128 and value.shape == key.shape,
                "K / V must be [N, H, 128]")
         self._call("fp_hbm_write", ctypes.byref(d), _dev(key, "key"), key.stride(0), key.stride(1),
                    _dev(value, "value"), value.stride(0), value.stride(1), _dev(slot_mapping, "slot_mapping"), n,
                    int(layer), _stream(key))
 
-    def hbm_encode(self, *args, ordered: bool = False) -> None:
+    def hbm_encode(self, *args, ordered: bool = False, desc: FpStore | None = None) -> None:
         """``ordered``: place each block's records in (kv, head) order
         (fp_hbm_encode_ordered) instead of by arrival."""
         state, (rank_of, layer, arena, page_bytes, max_close) = args[:13], args[13:]
         if int(max_close) == 0:
             return
-        d = _store_desc(state)
+        d = store_desc(state) if desc is None else desc
         _check(2 * int(max_close) <= state[6].numel(), "close list too small")
         _check(rank_of.numel() == d.num_layers * 2 * d.kv_heads * 256, "rank_of must hold every layer")
         _check(int(page_bytes) % 16 == 0 and int(page_bytes) < (1 << 31), "bad arena page size")
         self._call("fp_hbm_encode_ordered" if ordered else "fp_hbm_encode", ctypes.byref(d), _dev(rank_of, "rank_of"),
                    rank_of.numel(), int(layer), int(arena), int(page_bytes), int(max_close), _stream(rank_of))
 
-    def hbm_write_encode(self, *args, ordered: bool = False) -> None:
+    def hbm_write_encode(self, *args, ordered: bool = False, desc: FpStore | None = None) -> None:
         """hbm_write then hbm_encode of one layer in one launch
         (fp_hbm_write_encode); same arguments as the two calls."""
         state, (key, value, slot_mapping, rank_of, layer, arena, page_bytes, max_close) = args[:13], args[13:]
         n = key.size(0)
         if int(max_close) == 0:
-            self.hbm_write(*state, key, value, slot_mapping, layer)
+            self.hbm_write(*state, key, value, slot_mapping, layer, desc=desc)
             return
         if n == 0:
-            self.hbm_encode(*state, rank_of, layer, arena, page_bytes, max_close, ordered=ordered)
+            self.hbm_encode(*state, rank_of, layer, arena, page_bytes, max_close, ordered=ordered, desc=desc)
             return
         _check(key.stride(2) == 1 and value.stride(2) == 1, "head dim must be contiguous")
         _check(key.dtype == torch.bfloat16 and value.dtype == torch.bfloat16, "K / V must be BF16")
         _check(slot_mapping.dtype == torch.int64 and slot_mapping.numel() >= n, "slot_mapping must be int64 [N]")
-        d = _store_desc(state)
+        d = store_desc(state) if desc is None else desc
         _check(key.size(1) == d.kv_heads and key.size(2) == 128 and value.shape == key.shape,
                "K / V must be [N, H, 128]")
         _check(2 * int(max_close) <= state[6].numel(), "close list too small")
@@ -268,8 +272,8 @@ class Extension:
                    int(layer), _dev(rank_of, "rank_of"), rank_of.numel(), int(arena), int(page_bytes),
                    int(max_close), int(bool(ordered)), _stream(key))
 
-    def hbm_commit(self, *state) -> None:
-        d = _store_desc(state)
+    def hbm_commit(self, *state, desc: FpStore | None = None) -> None:
+        d = store_desc(state) if desc is None else desc
         self._call("fp_hbm_commit", ctypes.byref(d), _stream(state[0]))
 
     def hbm_gather(self, src_blocks, rec_addr, rec_len, plut, slut, wk, wv, kv_heads: int) -> None:
@@ -306,7 +310,7 @@ class Extension:
                    L, NB, H, _dev(out, "out"), out.numel(), int(stride), _dev(lengths, "lengths"), int(digest),
                    _stream(out))
 
-    def hbm_import(self, *args) -> None:
+    def hbm_import(self, *args, desc: FpStore | None = None) -> None:
         state = args[:13]
         src, offsets, blocks, status, arena_base, arena_stride, digest = args[13:]
         n = blocks.numel()
@@ -317,7 +321,7 @@ class Extension:
         _check(offsets.dtype == torch.int64 and offsets.numel() == n and blocks.dtype == torch.int32
                and status.dtype == torch.int32 and status.numel() >= n,
                "import metadata must be int64 offsets, int32 blocks / status")
-        d = _store_desc(state)
+        d = store_desc(state) if desc is None else desc
         _check(d.kv_heads <= 16, "too many KV heads")
         _check(arena_base.numel() == d.num_layers and arena_stride.numel() == d.num_layers,
                "arena tables must hold every layer")
@@ -434,4 +438,4 @@ def extension() -> Extension:
     return Extension(ctypes.CDLL(str(LIB_PATH)))
 
 
-__all__ = ["Extension", "FpStore", "LIB_PATH", "extension"]
+__all__ = ["Extension", "FpStore", "LIB_PATH", "extension", "store_desc"]
