@@ -15,6 +15,7 @@
 
 #include "../../include/fragpack_hip.h"
 #include "fp_capi_internal.hpp"
+#include "fp_page_claim.hpp"
 #include "fp_record.hpp"
 
 namespace fp {
@@ -1101,7 +1102,7 @@ __device__ __forceinline__ void enc_store(uint8_t* dst, const uint4 (&wd)[8], co
 // Persistent encoder: workgroup g encodes records r = g, g + grid, ... of
 // the n_closes * 2H records of this step (record r: kvh = r / n_closes of
 // block close_list[r % n_closes]) from staging into the block's arena page (each record
-// takes the next kDenseBytes + var_len bytes, claimed by CAS on fill), or raw
+// takes the next kDenseBytes + var_len bytes, claimed by an atomic add to fill), or raw
 // into the overflow pool when it does not code or no longer fits; and hands
 // the slot's record to the block's heir (hbm_kv.cu:262-429).  While record r
 // is encoded from registers, record r + grid streams from HBM straight into
@@ -1145,29 +1146,17 @@ __device__ __forceinline__ void stage_record(EncStage& st_buf, const uint8_t* sr
 // writes the page fill.
 enum EncMode { kEncClaim = 0, kEncBlockMajor = 1, kEncMeasure = 2, kEncPlaced = 3 };
 
-// The page offset of a record that added ``need`` to its block's fill and got
-// ``was`` back, or -1 if it spills.  An add that passes the page's end is taken
-// back; until then the fill reads past the page's end (and only then: it
-// holds at most the page otherwise), so another record that sees it so waits
-// for the true fill -- the one that added takes it back whatever happens --
-// and claims by compare-and-swap: it spills only if it does not fit beside the
-// records placed before it.
-__device__ __forceinline__ int page_claim(int32_t* fill, int was, int need, int64_t page_bytes, int& n_spill) {
-  if (was + need <= page_bytes) return was;
-  int cur = atomicSub(fill, need) - need;
-  for (;;) {
-    if (cur > page_bytes) {
-      cur = __hip_atomic_load(fill, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else if (cur + need <= page_bytes) {
-      const int prev = atomicCAS(fill, cur, cur + need);
-      if (prev == cur) return cur;
-      cur = prev;
-    } else {
-      ++n_spill;
-      return -1;
-    }
+// A block's page fill, as page_claim works on it.
+struct PageFill {
+  int32_t* fill;
+  __device__ __forceinline__ int sub(int n) const { return atomicSub(fill, n); }
+  __device__ __forceinline__ int load() const {
+    return __hip_atomic_load(fill, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-}
+  __device__ __forceinline__ int cas(int from, int to) const { return atomicCAS(fill, from, to); }
+};
+// what keeps claimed records apart: any two exceed any one
+static_assert(kDenseBytes + kVarCap < 2 * (kDenseBytes + kHeaderBytes), "page_claim's records could overlap");
 
 template <int kMode, bool kWrite>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kEncodeWgPerCu)))
@@ -1257,6 +1246,7 @@ encode_kernel(Store s, int layer, uint8_t* arena, int64_t page_bytes, const uint
   // one hot counter hit by every record serialises at its memory channel
   int n_enc = 0, n_fall = 0, n_err = 0, n_spill = 0;
   bool ovf_full = false;  // this workgroup found the overflow pool full
+  int page_polls = kPageWaitPolls;  // (thread 0) 0 once a fill stayed past its page's end
   int boff = 0;           // ordered encode: the block's next free page byte (thread 0)
   int r_next = r;
   for (int k = 0; r < n_rec; r = r_next, ++k) {
@@ -1384,7 +1374,10 @@ encode_kernel(Store s, int layer, uint8_t* arena, int64_t page_bytes, const uint
       const int need = kDenseBytes + res.var_len;
       if (tid == 0) cur = atomicAdd(fill, need);
       enc_var(wd, code, nib, sh, res, eo, ro);
-      if (tid == 0) sh.s_off = page_claim(fill, cur, need, page_bytes, n_spill);
+      if (tid == 0) {
+        sh.s_off = page_claim(PageFill{fill}, cur, need, page_bytes, page_polls);
+        n_spill += sh.s_off < 0;
+      }
     } else if (tid == 0) {
       sh.s_off = -1;
     }

@@ -728,6 +728,26 @@ def test_contended_pages_spill_only_what_does_not_fit(heads, fits):
     eng.check_gather()
 
 
+@pytest.mark.parametrize("fused", [False, True])
+def test_a_page_filled_past_its_end_spills_every_record(fused):
+    """A fill that rests past the page's end (as after pages of another size)
+    leaves no room: every record spills, the launch ends, the fill stays."""
+    eng = SimEngine(92, layers=1, heads=2, blocks=4, staging=2, overflow=16, fused=fused)
+    prepare = eng.store.prepare
+
+    def prepare_over_full_pages(*args):
+        prepare(*args)
+        eng.store.fill.fill_(eng.page + 16)
+
+    eng.store.prepare = prepare_over_full_pages
+    eng.step([("a", 3 * T)])
+    assert eng.check_records([0, 1, 2]) == (0, 3 * 2 * 2)
+    assert (eng.store.fill[0, :3] == eng.page + 16).all()
+    st = eng.store.stats()
+    assert (st.spills, st.encoded, st.err_overflow) == (12, 12, 0)
+    eng.check_gather()
+
+
 @pytest.mark.parametrize("n", [1023, 1024, 1025, 1100])
 def test_prepare_of_many_single_tokens(n):
     """Around one offset-0 token per thread of prepare's workgroup (its path
