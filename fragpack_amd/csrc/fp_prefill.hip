@@ -965,14 +965,19 @@ struct PfLaunch {
   int64_t steps;  // key tiles of all query tiles
   int waves;      // per workgroup
   int split_wgs;  // 0: not split
+  // the launch that does not split: heads of a grid row, rows, workgroups of a row
+  int head_sets;
+  int64_t rows, row_wgs;
 };
+// work items of a grid's x dimension (HIP's limit)
+constexpr int64_t kPfGridMost = (1LL << 32) - 1;
 
 PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
-                        int64_t max_seqlen_k) {
+                        int64_t max_seqlen_k, int64_t device) {
   const int64_t T = kPfRows / group;
   PfLaunch r;
   r.tiles = (max_seqlen_q + T - 1) / T;
-  const int64_t cus = device_cus() / kPfXcds * kPfXcds, steps = (max_seqlen_k + kPfKeys - 1) / kPfKeys;
+  const int64_t cus = device / kPfXcds * kPfXcds, steps = (max_seqlen_k + kPfKeys - 1) / kPfKeys;
   const int64_t most = r.tiles * num_seqs;
   const int64_t all = (total_q > 0 ? std::min(most, total_q / T + num_seqs) : most) * kv_heads;
   r.steps = all * steps;
@@ -981,6 +986,17 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   // in units of 0.1 us
   const bool split = all <= cus && 10 * (450 * cus + 23 * r.steps) < 9 * cus * (100 + 13 * steps);
   r.split_wgs = total_q > 0 && split && r.steps <= kPfSplitMost ? (int)cus : 0;
+  // The most head sets that divide the heads and that the grid's x dimension
+  // holds: a row has the query tiles of head_sets heads.
+  const int64_t items = most * (kPfWaves / r.waves);
+  for (r.head_sets = kPfXcds;; r.head_sets /= 2) {
+    const int64_t share = kPfXcds / r.head_sets;
+    r.rows = kv_heads / r.head_sets;
+    r.row_wgs = kPfXcds * ((items + share - 1) / share);
+    if (r.head_sets == 1 || (kv_heads % r.head_sets == 0 && r.row_wgs * 64 * r.waves <= kPfGridMost)) break;
+  }
+  // (with one head a row need not fill its last round over the XCDs)
+  if (r.row_wgs * 64 * r.waves > kPfGridMost) r.row_wgs = items;
   return r;
 }
 
@@ -996,8 +1012,22 @@ int64_t prefill_workspace(const PfLaunch& l) {
 extern "C" int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
                                               int64_t max_seqlen_q, int64_t max_seqlen_k) {
   if (kv_heads < 1 || group < 1 || kPfRows % group || num_seqs < 1 || total_q < 1 || max_seqlen_q < 1) return 0;
-  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k);
+  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, device_cus());
   return l.split_wgs ? prefill_workspace(l) : 0;
+}
+
+extern "C" int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
+                               int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t cus, int64_t* plan) {
+  FP_CHECK(plan && kv_heads >= 1 && group >= 1 && kPfRows % group == 0 && num_seqs >= 1 && total_q >= 0 &&
+               max_seqlen_q >= 1 && max_seqlen_k >= 0,
+           "bad prefill sizes");
+  const PfLaunch l =
+      prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, cus > 0 ? cus : device_cus());
+  plan[0] = l.waves;
+  plan[1] = l.split_wgs;
+  plan[2] = l.row_wgs;
+  plan[3] = l.rows;
+  return 0;
 }
 
 extern "C" int fp_prefill_attention(const void* q, int64_t q_stride, const void* wk, const void* wv, int64_t num_pages,
@@ -1048,17 +1078,11 @@ extern "C" int fp_prefill_attention_split(const void* q, int64_t q_stride, const
   p.group = (int)group;
   p.num_seqs = (int)num_seqs;
   p.tiles_per_seq = (int)tiles;
-  p.head_sets = 1;
-  for (int sets = kPfXcds; sets > 1; sets /= 2)
-    if (kv_heads % sets == 0 && tiles * num_seqs * sets < (1LL << 31)) {
-      p.head_sets = sets;
-      break;
-    }
   p.scale_log2 = (float)(scale * 1.4426950408889634);
   p.causal = causal ? 1 : 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // all LDS is static (two K and two V stages, 64 KB)
-  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k);
+  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, device_cus());
   if (workspace && l.split_wgs > 0) {
     const int64_t slots = 2 * (int64_t)l.split_wgs;
     FP_CHECK(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= prefill_workspace(l),
@@ -1077,8 +1101,9 @@ extern "C" int fp_prefill_attention_split(const void* q, int64_t q_stride, const
     hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)(l.split_wgs - 1), kPfWaves * kPfQt), dim3(kPfMergeThreads), 0,
                        s, p);
   } else {
-    const int64_t share = kPfXcds / p.head_sets, per_xcd = (tiles * num_seqs * (kPfWaves / l.waves) + share - 1) / share;
-    const dim3 grid((unsigned)(kPfXcds * per_xcd), (unsigned)(kv_heads / p.head_sets)), block(64 * l.waves);
+    FP_CHECK(l.row_wgs * 64 * l.waves <= kPfGridMost, "grid too large");
+    p.head_sets = l.head_sets;
+    const dim3 grid((unsigned)l.row_wgs, (unsigned)l.rows), block(64 * l.waves);
     if (l.waves == 4)
       hipLaunchKernelGGL((prefill_kernel<4, false>), grid, block, 0, s, p);
     else

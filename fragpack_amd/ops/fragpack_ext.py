@@ -134,6 +134,7 @@ class Extension:
             "fp_prefill_attention_split": [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64,
                                            _i64, _f64, _i32, _p, _i64, _p, _i64, _p],
             "fp_prefill_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _i64],
+            "fp_prefill_plan": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _p],
         }
         for name, args in sigs.items():
             fn = getattr(lib, name)

@@ -292,6 +292,15 @@ int fp_prefill_attention_split(const void* q, int64_t q_stride, const void* wk, 
 /* Workspace bytes of fp_prefill_attention_split (0: none is used). */
 int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
                                    int64_t max_seqlen_q, int64_t max_seqlen_k);
+/*
+ * What a call of these sizes launches on a device of ``cus`` compute units (0:
+ * the current one), without launching it: plan[0] waves per workgroup, plan[1]
+ * workgroups of the split launch that a workspace allows (0: none), plan[2]
+ * and plan[3] workgroups of a row and rows of the grid otherwise.  total_q 0:
+ * as fp_prefill_attention.
+ */
+int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
+                    int64_t max_seqlen_k, int64_t cus, int64_t* plan);
 
 #ifdef __cplusplus
 }

@@ -121,6 +121,23 @@ def test_workgroup_mapping(heads, q_lens):
     _run(50 + heads, heads=heads, group=2, q_lens=q_lens, k_lens=[n + 40 * (i % 2) for i, n in enumerate(q_lens)])
 
 
+def test_a_grid_past_one_row_of_every_head():
+    # 4 sequences bounded by 2^23 queries: 2^20 tiles a head, nearly all dead;
+    # all 8 heads in one grid row would pass the 2^32 work items a launch takes
+    import torch
+
+    from fragpack_amd.ops.prefill_attn import flash_attn_varlen_func
+
+    q, wk, wv, bt, cu, kl = (torch.from_numpy(x) if isinstance(x, np.ndarray) else x
+                             for x in _case(61, 8, 8, [40, 1, 0, 33], [40, 130, 0, 33]))
+    out = torch.full_like(q, float("nan"), device="cuda")
+    print("prefill with 2^20 tiles a head", flush=True)
+    flash_attn_varlen_func(q=q.cuda(), k=wk.cuda(), v=wv.cuda(), out=out, cu_seqlens_q=cu.cuda(), max_seqlen_q=1 << 23,
+                           seqused_k=kl.cuda(), max_seqlen_k=130, block_table=bt.cuda())
+    ref = _reference(q, wk, wv, bt.numpy(), cu.numpy(), kl.numpy(), 8, D ** -0.5, True)
+    torch.testing.assert_close(out.float().cpu(), ref, atol=ATOL, rtol=RTOL)
+
+
 # Grids with fewer query tiles than CUs split their keys over the CUs
 # (fp_prefill_attention_split): P rounds as in the unsplit launch and only the
 # order of fp32 sums differs, so a BF16 output moves by at most one step

@@ -214,3 +214,25 @@ def test_plan_reuse_without_a_plan_is_refused():
     ws[2]._fp_plan_key = (units + 1, B, H)
     with pytest.raises(RuntimeError, match="plan first"):
         extension().fused_decode(*args, False, 0.1, G)
+
+
+def prefill_plan(heads, group, seqs, total_q, max_q, max_k, cus=256):
+    """(waves, split workgroups, workgroups of a row, rows) of a prefill call on ``cus`` compute units."""
+    lib = ctypes.CDLL(str(LIB_PATH))
+    lib.fp_prefill_plan.argtypes = [ctypes.c_int64] * 7 + [ctypes.c_void_p]
+    plan = (ctypes.c_int64 * 4)()
+    assert lib.fp_prefill_plan(heads, group, seqs, total_q, max_q, max_k, cus, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.parametrize("heads", [1, 2, 4, 5, 6, 8, 12, 16, 64])
+@pytest.mark.parametrize("seqs,tiles", [(1, 1), (3, 11), (4, 1 << 18), (512, 2048), (8, (1 << 20) - 1), (1, (1 << 23) - 1)])
+def test_prefill_grid_covers_the_tiles_within_the_launch_limit(heads, seqs, tiles):
+    """HIP takes fewer than 2^32 work items along x: one head's tiles fit up to
+    2^23 - 1 workgroups of 512, so that many are never refused, and the rows
+    hold every (query tile, head)."""
+    waves, _, row, rows = prefill_plan(heads, 8, seqs, 0, 32 * tiles, 4096)
+    assert row * 64 * waves < 1 << 32
+    assert rows <= heads and heads % rows == 0
+    per_head = seqs * tiles * (8 // waves)
+    assert per_head * (heads // rows) <= row < per_head * (heads // rows) + 8 * (heads // rows)
