@@ -959,6 +959,12 @@ namespace {
 //   longest query tile by 10%: 200 new tokens over 8192 at H 4, G 8 take 76 us
 //   instead of 175 (4 waves) or 226 (8).
 constexpr int64_t kPfSplitMost = 1 << 16;  // key tiles (1 KB of workspace each)
+// The rule in units of 0.1 us, kPfSplitMargin tenths: its own time, per key tile
+// of a CU's share, and of the launch that does not split: its own, per key tile.
+constexpr int64_t kPfSplitBase = 450, kPfSplitStep = 23, kPfWholeBase = 100, kPfWholeStep = 13, kPfSplitMargin = 9;
+// The fewest key tiles of the longest query tile for which it can hold.
+constexpr int64_t kPfSplitSteps =
+    (10 * kPfSplitBase - kPfSplitMargin * kPfWholeBase) / (kPfSplitMargin * kPfWholeStep) + 1;
 
 struct PfLaunch {
   int64_t tiles;  // query tiles of the longest sequence
@@ -983,8 +989,8 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   r.steps = all * steps;
   const bool fresh = 2 * max_seqlen_k <= 3 * max_seqlen_q;
   r.waves = 4 * all <= 3 * cus || (fresh && all <= 4 * cus) ? 4 : kPfWaves;
-  // in units of 0.1 us
-  const bool split = all <= cus && 10 * (450 * cus + 23 * r.steps) < 9 * cus * (100 + 13 * steps);
+  const bool split = all <= cus && 10 * (kPfSplitBase * cus + kPfSplitStep * r.steps) <
+                                      kPfSplitMargin * cus * (kPfWholeBase + kPfWholeStep * steps);
   r.split_wgs = total_q > 0 && split && r.steps <= kPfSplitMost ? (int)cus : 0;
   // The most head sets that divide the heads and that the grid's x dimension
   // holds: a row has the query tiles of head_sets heads.
@@ -1015,6 +1021,8 @@ extern "C" int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, i
   const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, device_cus());
   return l.split_wgs ? prefill_workspace(l) : 0;
 }
+
+extern "C" int64_t fp_prefill_split_min_keys(void) { return (kPfSplitSteps - 1) * kPfKeys + 1; }
 
 extern "C" int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
                                int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t cus, int64_t* plan) {

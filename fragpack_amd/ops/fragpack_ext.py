@@ -134,6 +134,7 @@ class Extension:
             "fp_prefill_attention_split": [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64,
                                            _i64, _f64, _i32, _p, _i64, _p, _i64, _p],
             "fp_prefill_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _i64],
+            "fp_prefill_split_min_keys": [],
             "fp_prefill_plan": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _p],
         }
         for name, args in sigs.items():
@@ -141,6 +142,8 @@ class Extension:
             fn.argtypes = args
             fn.restype = _i32
         lib.fp_prefill_workspace_bytes.restype = _i64
+        lib.fp_prefill_split_min_keys.restype = _i64
+        self._split_keys = lib.fp_prefill_split_min_keys()  # shorter contexts need no workspace query
         self._fused = lib.fp_fused_decode
         self._fused_append = lib.fp_fused_decode_append
         lib.fp_last_error.restype = ctypes.c_char_p
@@ -409,11 +412,10 @@ class Extension:
         _check(block_table.dtype == i32 and len(bsh) == 2 and bst[1] == 1
                and bsh[0] == n_seqs, "block_table must be int32 [B, pages] with contiguous rows")
         # Workspace for the parts of split query tiles: from the caching
-        # allocator, so ordered with this stream's work and private to the call
-        # (contexts of up to 30 key tiles never split: no need to ask).
+        # allocator, so ordered with this stream's work and private to the call.
         n, max_q, max_k = qsh[0], int(max_seqlen_q), int(max_seqlen_k)
         ws, ws_bytes = None, 0
-        if max_k > 1920:
+        if max_k >= self._split_keys:
             ws_bytes = self._lib.fp_prefill_workspace_bytes(kvh, group, n_seqs, n, max_q, max_k)
             if ws_bytes:
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)

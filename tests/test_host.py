@@ -236,3 +236,20 @@ def test_prefill_grid_covers_the_tiles_within_the_launch_limit(heads, seqs, tile
     assert rows <= heads and heads % rows == 0
     per_head = seqs * tiles * (8 // waves)
     assert per_head * (heads // rows) <= row < per_head * (heads // rows) + 8 * (heads // rows)
+
+
+def test_no_call_below_the_split_key_bound_splits():
+    """The bound below which a caller need not ask for a workspace is the
+    launch rule's own: nothing below it splits, one row a key tile past it does."""
+    from fragpack_amd.ops.fragpack_ext import extension
+
+    ext = extension()
+    least = ext._lib.fp_prefill_split_min_keys()
+    assert ext._split_keys == least and prefill_plan(1, 8, 1, 1, 1, least + 64)[1] == 256
+    rng = np.random.default_rng(5)
+    for _ in range(2000):
+        heads, group, seqs = int(rng.integers(1, 33)), int(2 ** rng.integers(0, 4)), int(rng.integers(1, 9))
+        max_q = int(np.exp(rng.uniform(0, 9)))
+        total = int(rng.integers(max_q, seqs * max_q + 1))
+        assert prefill_plan(heads, group, seqs, total, max_q, int(rng.integers(1, least)))[1] == 0
+        assert prefill_plan(heads, group, seqs, 0, max_q, 1 << 20)[1] == 0  # no rows given: never split
