@@ -1022,6 +1022,15 @@ extern "C" int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, i
   return l.split_wgs ? prefill_workspace(l) : 0;
 }
 
+extern "C" int64_t fp_prefill_workspace_most(int64_t max_seqlen_k, int64_t cus) {
+  const int64_t steps = (max_seqlen_k + kPfKeys - 1) / kPfKeys;
+  if (steps < kPfSplitSteps) return 0;
+  PfLaunch l{};
+  l.split_wgs = (int)((cus > 0 ? cus : device_cus()) / kPfXcds * kPfXcds);
+  l.steps = std::min(steps * l.split_wgs, kPfSplitMost);  // a split call has at most a query tile per CU
+  return prefill_workspace(l);
+}
+
 extern "C" int64_t fp_prefill_split_min_keys(void) { return (kPfSplitSteps - 1) * kPfKeys + 1; }
 
 extern "C" int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,

@@ -241,6 +241,7 @@ class FragPackMetadata:
     prefills: list[PrefillGroup]
     wk: object
     wv: object
+    split_workspace: object = None
 
 
 class FragPackRunner:
@@ -277,6 +278,7 @@ class FragPackRunner:
     ) -> None:
         import torch
 
+        from fragpack_amd.ops.fragpack_ext import extension
         from fragpack_amd.ops.fused_attn_decode import decode_units, workspace_elems
 
         self.kv_heads = kv_heads
@@ -302,6 +304,12 @@ class FragPackRunner:
         shape = (self.workspace_pages, BLOCK_TOKENS, kv_heads, HEAD_DIM)
         self.wk = torch.empty(shape, dtype=torch.bfloat16, device=self.device)
         self.wv = torch.empty(shape, dtype=torch.bfloat16, device=self.device)
+        # parts of the prefill calls that split their keys over the CUs (any
+        # call of up to max_model_len keys): a full device then refuses the
+        # runner, not a prefill in mid-serving
+        with torch.cuda.device(self.device):
+            split_bytes = extension().prefill_workspace_bytes(max_model_len)
+        self.split_workspace = torch.empty(split_bytes, dtype=torch.uint8, device=self.device)
         self.store = None
         self.store_key: tuple[int, int] | None = None
         self.layer_tables: list = []
@@ -332,6 +340,7 @@ class FragPackRunner:
         self.layer_tables = [RecordTables(*store.layer_tables(i)) for i in range(len(caches))]
         memory = store.memory_usage()
         memory["prefill_workspace"] = sum(t.numel() * t.element_size() for t in (self.wk, self.wv))
+        memory["prefill_split_workspace"] = self.split_workspace.nbytes
         memory["decode_workspace"] = sum(t.numel() * t.element_size() for t in self.decode_workspace)
         raw = 2 * self.kv_heads * BLOCK_TOKENS * HEAD_DIM * 2
         publish_capacity(FragPackCapacity(blocks=store.num_blocks, block_tokens=BLOCK_TOKENS, layers=store.num_layers,
@@ -420,6 +429,7 @@ class FragPackRunner:
             prefills=prefills,
             wk=self.wk,
             wv=self.wv,
+            split_workspace=self.split_workspace,
         )
 
 
@@ -447,7 +457,7 @@ def layer_forward(md: FragPackMetadata, li: int, query, key, value, output, scal
         ``output``.
     """
     from fragpack_amd.ops.fused_attn_decode import decode_attention
-    from fragpack_amd.ops.prefill_attn import flash_attn_varlen_func
+    from fragpack_amd.ops.prefill_attn import prefill_attention
 
     if md is None:
         return output.zero_()
@@ -467,10 +477,9 @@ def layer_forward(md: FragPackMetadata, li: int, query, key, value, output, scal
                          md.units, output[:nd], md.decode_workspace, replan=li == 0)
     for g in md.prefills:
         store.gather(li, g.src_blocks, md.wk, md.wv)
-        flash_attn_varlen_func(q=query[g.tok0 : g.tok1], k=md.wk, v=md.wv, out=output[g.tok0 : g.tok1],
-                               cu_seqlens_q=g.cu_seqlens_q, max_seqlen_q=g.max_seqlen_q, seqused_k=g.seqused_k,
-                               max_seqlen_k=g.max_seqlen_k, softmax_scale=scale, causal=True,
-                               block_table=g.block_table)
+        prefill_attention(query[g.tok0 : g.tok1], md.wk, md.wv, output[g.tok0 : g.tok1], g.cu_seqlens_q,
+                          g.max_seqlen_q, g.seqused_k, g.max_seqlen_k, scale, True, g.block_table,
+                          workspace=md.split_workspace)
     if not fused:
         store.encode(li, md.max_close)
     if li == md.last_layer:

@@ -134,6 +134,7 @@ class Extension:
             "fp_prefill_attention_split": [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64,
                                            _i64, _f64, _i32, _p, _i64, _p, _i64, _p],
             "fp_prefill_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _i64],
+            "fp_prefill_workspace_most": [_i64, _i64],
             "fp_prefill_split_min_keys": [],
             "fp_prefill_plan": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _p],
         }
@@ -142,6 +143,7 @@ class Extension:
             fn.argtypes = args
             fn.restype = _i32
         lib.fp_prefill_workspace_bytes.restype = _i64
+        lib.fp_prefill_workspace_most.restype = _i64
         lib.fp_prefill_split_min_keys.restype = _i64
         self._split_keys = lib.fp_prefill_split_min_keys()  # shorter contexts need no workspace query
         self._fused = lib.fp_fused_decode
@@ -390,7 +392,11 @@ class Extension:
 
     # -- prefill (the FlashAttention call of backend.py:560-575) --
     def prefill_attention(self, q, wk, wv, out, cu_seqlens_q, seqused_k, block_table, max_seqlen_q: int,
-                          max_seqlen_k: int, scale: float, causal: bool) -> None:
+                          max_seqlen_k: int, scale: float, causal: bool,
+                          workspace: torch.Tensor | None = None) -> None:
+        """``workspace``: uint8 device memory for the parts of a split call
+        (prefill_workspace_bytes(max_k) holds every call's), not shared with a
+        call that may overlap; None: allocated by the call where it splits."""
         # one tuple read per tensor property: short calls are bound by the host
         qsh, qst, osh, ost, ksh = q.shape, q.stride(), out.shape, out.stride(), wk.shape
         bsh, bst, bf16, i32 = block_table.shape, block_table.stride(), torch.bfloat16, torch.int32
@@ -411,19 +417,37 @@ class Extension:
                and cu_seqlens_q.numel() == n_seqs + 1, "cu_seqlens_q int32 [B + 1], seqused_k int32 [B]")
         _check(block_table.dtype == i32 and len(bsh) == 2 and bst[1] == 1
                and bsh[0] == n_seqs, "block_table must be int32 [B, pages] with contiguous rows")
-        # Workspace for the parts of split query tiles: from the caching
-        # allocator, so ordered with this stream's work and private to the call.
         n, max_q, max_k = qsh[0], int(max_seqlen_q), int(max_seqlen_k)
         ws, ws_bytes = None, 0
         if max_k >= self._split_keys:
             ws_bytes = self._lib.fp_prefill_workspace_bytes(kvh, group, n_seqs, n, max_q, max_k)
             if ws_bytes:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+                ws = self._split_workspace(workspace, ws_bytes, q.device)
+                if ws is None:
+                    ws_bytes = 0
         self._call("fp_prefill_attention_split", _dev(q, "q"), qst[0], _dev(wk, "k"), _dev(wv, "v"), ksh[0], kvh,
                    group, _dev(cu_seqlens_q, "cu_seqlens_q"), _dev(seqused_k, "seqused_k"),
                    _dev(block_table, "block_table"), bst[0], n_seqs, n, max_q, max_k, float(scale),
                    int(bool(causal)), _dev(out, "out"), ost[0], ws.data_ptr() if ws_bytes else None, ws_bytes,
                    _stream(q))
+
+    def prefill_workspace_bytes(self, max_seqlen_k: int) -> int:
+        """Bytes of a workspace that serves any prefill call of up to
+        ``max_seqlen_k`` keys on the current device."""
+        return self._lib.fp_prefill_workspace_most(int(max_seqlen_k), 0)
+
+    @staticmethod
+    def _split_workspace(given: torch.Tensor | None, need: int, device: torch.device) -> torch.Tensor | None:
+        """The caller's workspace, else one from the caching allocator (ordered
+        with the stream's work, private to the call), else None: a device too
+        full for it runs the launch that needs none."""
+        if (given is not None and given.device == device and given.is_contiguous() and given.nbytes >= need
+                and given.data_ptr() % 16 == 0):
+            return given
+        try:
+            return torch.empty(need, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            return None
 
 
 @functools.cache

@@ -8,8 +8,8 @@ workspace that ``HbmKvStore.gather`` fills
                            cu_seqlens_q=..., max_seqlen_q=..., seqused_k=..., max_seqlen_k=...,
                            softmax_scale=scale, causal=True, block_table=..., fa_version=...)
 
-Here the same call runs a hand-written gfx950 MFMA kernel
-(``fp_prefill_attention``).  Semantics follow FlashAttention's varlen
+Here the same call runs hand-written gfx950 MFMA kernels
+(``fp_prefill_attention_split``).  Semantics follow FlashAttention's varlen
 contract for a paged KV cache: sequence b has ``cu_seqlens_q[b+1] -
 cu_seqlens_q[b]`` queries, which are its last positions, over
 ``seqused_k[b]`` keys (causal mask aligned bottom-right); key j of b is row
@@ -61,16 +61,46 @@ def flash_attn_varlen_func(
 
     Async/thread-safety:
         Enqueues on the current stream; not synchronized.
+
+    A call with few query tiles over long contexts splits its keys over the
+    GPU and takes up to ~140 MB for the parts from torch's allocator for its
+    duration (without that much free it runs unsplit); a caller with a
+    workspace of its own uses :func:`prefill_attention`.
     """
     del fa_version
+    return prefill_attention(q, k, v, out, cu_seqlens_q, max_seqlen_q, seqused_k, max_seqlen_k, softmax_scale, causal,
+                             block_table)
+
+
+def prefill_attention(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    out: torch.Tensor | None,
+    cu_seqlens_q: torch.Tensor | None,
+    max_seqlen_q: int,
+    seqused_k: torch.Tensor | None,
+    max_seqlen_k: int,
+    softmax_scale: float | None,
+    causal: bool,
+    block_table: torch.Tensor | None,
+    workspace: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """:func:`flash_attn_varlen_func` with the caller's workspace.
+
+    Args:
+        workspace: uint8 device memory of ``extension().prefill_workspace_bytes
+            (max_seqlen_k)`` for a split call's parts, which no overlapping
+            call uses; None or too small: allocated by the call if it splits.
+    """
     if cu_seqlens_q is None or seqused_k is None or block_table is None:
         raise ValueError("cu_seqlens_q, seqused_k and block_table are required (paged varlen form)")
     if out is None:
         out = torch.empty_like(q)
     scale = softmax_scale if softmax_scale is not None else q.size(-1) ** -0.5
     extension().prefill_attention(q, k, v, out, cu_seqlens_q, seqused_k, block_table, max_seqlen_q, max_seqlen_k,
-                                  scale, causal)
+                                  scale, causal, workspace=workspace)
     return out
 
 
-__all__ = ["flash_attn_varlen_func"]
+__all__ = ["flash_attn_varlen_func", "prefill_attention"]

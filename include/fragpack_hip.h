@@ -292,6 +292,12 @@ int fp_prefill_attention_split(const void* q, int64_t q_stride, const void* wk, 
 /* Workspace bytes of fp_prefill_attention_split (0: none is used). */
 int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
                                    int64_t max_seqlen_q, int64_t max_seqlen_k);
+/*
+ * The most that fp_prefill_workspace_bytes asks for in any call of up to
+ * max_seqlen_k keys on a device of ``cus`` compute units (0: the current one):
+ * for a caller that keeps one workspace.
+ */
+int64_t fp_prefill_workspace_most(int64_t max_seqlen_k, int64_t cus);
 /* The max_seqlen_k below which no call uses a workspace. */
 int64_t fp_prefill_split_min_keys(void);
 /*

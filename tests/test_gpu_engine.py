@@ -246,3 +246,39 @@ def test_engine_steps_match_fp32_attention(driver, monkeypatch, tmp_path):
     cap = get_capacity()
     assert cap is not None and cap.blocks == NB and cap.layers == L and cap.kv_heads == H
     assert cap.memory["arena"] == NB * L * cap.page_bytes
+
+
+def test_a_layer_allocates_nothing(monkeypatch):
+    """A step's layers run in what the runner holds and publishes: a short
+    chunk over a long context (the split prefill) allocates no device memory."""
+    import torch
+
+    from fragpack_amd.compression.attn_tables import device_tables
+    from fragpack_amd.integrations.vllm.capacity import get_capacity
+    from fragpack_amd.integrations.vllm.step import FragPackRunner, layer_forward
+    from fragpack_amd.ops.fragpack_ext import extension
+    from fragpack_amd.ops.hbm_kv import page_bytes
+
+    ctx, chunk, pages = 4096, 64, 40
+    rng = np.random.default_rng(63)
+    tables = workloads.calibrated_tables(rng, H, workloads.channel_scales(rng, H, 0.02))
+    caches = [torch.empty((pages, page_bytes(H)), dtype=torch.uint8, device="cuda")]
+    runner = FragPackRunner(H, device_tables(tables, torch.device("cuda")), "cuda", ctx, 1, ctx + chunk, 64)
+    table = torch.arange(pages, dtype=torch.int32, device="cuda")[None]
+    gen = torch.Generator(device="cuda").manual_seed(64)
+    done = 0
+    for n in (ctx, chunk):
+        kv = torch.randn((2, n, H, D), generator=gen, device="cuda").to(torch.bfloat16)
+        q = torch.randn((n, H * G, D), generator=gen, device="cuda").to(torch.bfloat16)
+        out = torch.empty_like(q)
+        seq = np.array([done + n])
+        md = runner.build(caches, np.array([0, n]), seq, torch.tensor(seq, dtype=torch.int32, device="cuda"), table,
+                          torch.arange(done, done + n, device="cuda"), np.zeros(0, np.int32))
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        layer_forward(md, 0, q, kv[0], kv[1], out, D ** -0.5)
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before, n
+        done += n
+    assert extension()._lib.fp_prefill_workspace_bytes(H, G, 1, chunk, chunk, ctx + chunk) > 0
+    assert torch.isfinite(out).all()
+    assert get_capacity().memory["prefill_split_workspace"] == extension().prefill_workspace_bytes(ctx + chunk) > 0

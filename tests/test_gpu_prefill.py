@@ -201,6 +201,47 @@ def test_split_matches_unsplit(heads, group, q_lens, k_lens, causal):
         torch.testing.assert_close(outs[1].cpu(), ref, atol=ATOL, rtol=RTOL)
 
 
+def test_split_workspace_from_the_caller_or_none_at_all(monkeypatch):
+    """The caller's workspace is used in place of one from the allocator (same
+    bits, no allocation); a device too full for one runs the launch that needs
+    none."""
+    import torch
+
+    from fragpack_amd.ops.fragpack_ext import extension
+    from fragpack_amd.ops.prefill_attn import prefill_attention
+
+    ext = extension()
+    q, wk, wv, bt, cu, kl = (torch.from_numpy(x).cuda() if isinstance(x, np.ndarray) else x.cuda()
+                             for x in _case(81, 2, 4, [120, 1], [4000, 2500]))
+    assert ext._lib.fp_prefill_workspace_bytes(2, 4, 2, 121, 120, 4000) > 0
+
+    def run(out, workspace=None):
+        return prefill_attention(q, wk, wv, out, cu, 120, kl, 4000, None, True, bt, workspace=workspace)
+
+    want = run(torch.empty_like(q))
+    ws = torch.empty(ext.prefill_workspace_bytes(4000), dtype=torch.uint8, device="cuda")
+    got, small, plain = (torch.full_like(q, float("nan")) for _ in range(3))
+    whole = torch.full_like(q, float("nan"))
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: pytest.fail("allocated in the call"))
+    run(got, ws)
+    assert torch.equal(got, want)
+
+    def full(*a, **k):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(torch, "empty", full)
+    run(small, ws[: ws.numel() // 64])  # too small: as without one
+    run(plain)
+    monkeypatch.setattr(torch, "empty", empty)
+    rc = ext._lib.fp_prefill_attention(q.data_ptr(), q.stride(0), wk.data_ptr(), wv.data_ptr(), wk.shape[0], 2, 4,
+                                       cu.data_ptr(), kl.data_ptr(), bt.data_ptr(), bt.stride(0), 2, 120, 4000,
+                                       D ** -0.5, 1, whole.data_ptr(), whole.stride(0),
+                                       torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(plain, whole) and torch.equal(small, whole)
+
+
 @pytest.mark.parametrize("heads,group,q_lens,k_lens", [
     (2, 1, [100, 300], [100, 500]),  # shares of a query tile are token ranges
     (3, 2, [129, 1, 128], [300, 70, 128]),

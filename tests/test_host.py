@@ -253,3 +253,24 @@ def test_no_call_below_the_split_key_bound_splits():
         total = int(rng.integers(max_q, seqs * max_q + 1))
         assert prefill_plan(heads, group, seqs, total, max_q, int(rng.integers(1, least)))[1] == 0
         assert prefill_plan(heads, group, seqs, 0, max_q, 1 << 20)[1] == 0  # no rows given: never split
+
+
+def test_one_workspace_serves_every_split_call():
+    """The largest workspace of any call of up to max_k keys holds what each
+    such call asks for: the sizes here are the library's for 256 CUs, whose
+    part slots and key-tile entries are 2 x 133120 + 32 and 1032 bytes."""
+    lib = ctypes.CDLL(str(LIB_PATH))
+    i64 = ctypes.c_int64
+    lib.fp_prefill_workspace_most.argtypes, lib.fp_prefill_workspace_most.restype = [i64, i64], i64
+    lib.fp_prefill_split_min_keys.restype = i64
+    assert lib.fp_prefill_workspace_most(lib.fp_prefill_split_min_keys() - 1, 256) == 0
+    rng = np.random.default_rng(6)
+    for _ in range(2000):
+        heads, group, seqs = int(rng.integers(1, 33)), int(2 ** rng.integers(0, 4)), int(rng.integers(1, 5))
+        max_q, max_k = int(np.exp(rng.uniform(0, 8))), int(np.exp(rng.uniform(7.5, 13)))
+        total = int(rng.integers(max_q, seqs * max_q + 1))
+        if prefill_plan(heads, group, seqs, total, max_q, max_k)[1]:
+            rows = 256 // group
+            tiles = min(seqs * -(-max_q // rows), total // rows + seqs) * heads
+            need = 256 * (2 * 133120 + 32) + tiles * -(-max_k // 64) * 1032
+            assert need <= lib.fp_prefill_workspace_most(max_k, 256)
