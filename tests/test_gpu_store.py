@@ -763,6 +763,44 @@ def test_prepare_of_many_single_tokens(n):
     eng.step([("n%d" % i, 1) for i in range(150)] + [("m%d" % i, 1) for i in range(40)], pad=3)
 
 
+def test_prepare_releases_many_slots_over_many_blocks():
+    """Blocks past the first GC round (8192) and more released slots than
+    prepare keeps in LDS (2048): the next claims pop them from the stack."""
+    eng = SimEngine(11, layers=1, heads=1, blocks=9400, staging=2100, overflow=8, max_tokens=2200)
+    eng.pool = list(range(7100, 9400))  # on both sides of block 8192
+    names = [str(i) for i in range(2090)]
+    eng.step([(x, 1) for x in names])
+    for x in names:
+        eng.finish(x)
+    eng.step([("n%d" % i, 1) for i in range(900)])
+    eng.step([("n%d" % i, 1) for i in range(900)])
+
+
+@pytest.mark.parametrize("n", [5, 1030])
+def test_prepare_of_more_blocks_than_its_bitmaps_hold(n):
+    eng = SimEngine(13, layers=1, heads=1, blocks=65536 + 1200, page=2 * DENSE, staging=40, overflow=64, max_tokens=2 * n * T)
+    eng.pool = list(range(65536 - 40, 65536 + 1200))
+    eng.step([("a", 17), ("b", 3 * T)])
+    eng.step([("a", T)] + [("m%d" % i, 1) for i in range(n)] if n < 40 else [("a", T), ("c", n * T + 3)])
+    eng.finish("b")
+    eng.step([("a", 1), ("d", 2 * T + 1)])
+
+
+@pytest.mark.parametrize("reqs", [1, 70])
+def test_prepare_of_steps_that_open_and_close_nothing(reqs):
+    """Decode steps between blocks: nothing to list, but slots of finished
+    requests still go back; then steps that only open or only close."""
+    eng = SimEngine(17 + reqs, layers=1, heads=1, blocks=2 * reqs + 4, staging=reqs, overflow=8)
+    names = [str(i) for i in range(reqs)]
+    eng.step([(x, T - 2) for x in names[:1]] + [(x, 3) for x in names[1:]])
+    eng.step([(x, 1) for x in names])  # nothing opens or closes
+    for x in names[1::2]:
+        eng.finish(x)
+    eng.step([(names[0], 1)] + [(x, 1) for x in names[2::2]])  # closes one
+    eng.step([(x, 1) for x in names[2::2]] or [(names[0], 1)])  # nothing, after a close
+    eng.step([(names[0], 1)])  # opens one
+
+
 def test_prepare_of_a_step_with_more_closes_than_threads():
     n = 1030
     eng = SimEngine(5, layers=1, heads=1, blocks=n + 40, staging=4, overflow=8, max_tokens=(n + 2) * T)
