@@ -274,19 +274,14 @@ __device__ __forceinline__ void load_slab(rsrc_t r, bool raw, int slab, int nt, 
   b.v[5] = make_uint4(s2.x, s2.y, s3.x, s3.y);
 }
 
-// Loads thread ``t``'s (0..255) dense data of a record.
-__device__ __forceinline__ void load_thread(const uint8_t* rec, bool raw, int t, SlabBuf& b) {
+// Loads thread ``t``'s (0..255) dense data of a coded record.
+__device__ __forceinline__ void load_thread(const uint8_t* rec, int t, SlabBuf& b) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) b.v[j] = ld16_nt(rec + 16 * (256 * j + t));
-  if (raw) {
-    b.v[4] = ld16_nt(rec + 16 * (256 * 4 + t));
-    b.v[5] = ld16_nt(rec + 16 * (256 * 5 + t));
-  } else {
-    const uint2 s0 = ld8_nt(rec + kLowBytes + 8 * t), s1 = ld8_nt(rec + kLowBytes + 8 * (256 + t));
-    const uint2 s2 = ld8_nt(rec + kLowBytes + 8 * (512 + t));
-    b.v[4] = make_uint4(s0.x, s0.y, s1.x, s1.y);
-    b.v[5] = make_uint4(s2.x, s2.y, 0u, 0u);
-  }
+  const uint2 s0 = ld8_nt(rec + kLowBytes + 8 * t), s1 = ld8_nt(rec + kLowBytes + 8 * (256 + t));
+  const uint2 s2 = ld8_nt(rec + kLowBytes + 8 * (512 + t));
+  b.v[4] = make_uint4(s0.x, s0.y, s1.x, s1.y);
+  b.v[5] = make_uint4(s2.x, s2.y, 0u, 0u);
 }
 
 __device__ __forceinline__ uint32_t u4(const uint4& v, int i) {
@@ -406,9 +401,18 @@ __device__ __forceinline__ void raw_tail(const SlabBuf& b, uint4 w6, uint4 w7, E
   emit(std::integral_constant<int, 7>{}, w7);
 }
 
+// Thread ``t``'s (0..255) words of a raw record, the last two loaded behind the
+// first (1024 raw records 13.7 us, 14.8 with all eight at once).
 template <typename Emit>
-__device__ __forceinline__ void raw_words(const SlabBuf& b, const uint8_t* rec, int t, Emit&& emit) {
-  raw_tail(b, ld16_nt(rec + 16 * (256 * 6 + t)), ld16_nt(rec + 16 * (256 * 7 + t)), emit);
+__device__ __forceinline__ void raw_words(const uint8_t* rec, int t, Emit&& emit) {
+  uint4 wd[8];
+#pragma unroll
+  for (int st = 0; st < 6; ++st) wd[st] = ld16_nt(rec + 16 * (256 * st + t));
+  static_for<0, 2>([&](auto st) { emit(st, wd[decltype(st)::value]); });
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int st = 6; st < 8; ++st) wd[st] = ld16_nt(rec + 16 * (256 * st + t));
+  static_for<2, 8>([&](auto st) { emit(st, wd[decltype(st)::value]); });
 }
 
 template <typename Emit>

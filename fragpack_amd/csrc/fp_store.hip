@@ -1498,8 +1498,10 @@ constexpr int kTileRow = 256;  // bytes per token row in the tile
 // (36.9 KB: four workgroups per CU; with an escape area per wave it was 49 KB
 // and three, and a 64-block H 8 gather's 1024 workgroups took two rounds.
 // With that, and the variable region in flight beside the dense part instead
-// of read header first, 64 blocks take 11.6 us, 15.6 before; 256 blocks 47.6,
-// 50.7 before: 4.8 TB/s read and written, what a copy reaches.)
+// of read header first, cold records (H 8): 1 block 5.2 us, 5.4 before; 16
+// blocks 6.2, 6.5; 64 blocks 10.9, 16.4; 128 blocks 24.2, 28.2: 4.8 TB/s read
+// and written, what a copy reaches.  512 to 768 raw records lose: 48 all-raw
+// blocks 10.3, 9.2 before; 8 of them 4.5, 4.7; 64 13.7, 15.1.)
 struct DecShared {
   uint8_t tile[kTokens * kTileRow];
   uint8_t esc[kEscLds];  // the record's expanded escape bytes, by ordinal
@@ -1530,17 +1532,20 @@ __device__ void decode_record_to_tile(const uint8_t* rec, int vlen, int kv, cons
     }
   };
   auto emit = [&](auto st, const uint4& wd) { put(decltype(st)::value, wd); };
-  SlabBuf b;
-  const bool raw = vlen > kVarCap;
-  // the thread's 8 bytes of the variable region go out with its dense loads
-  const int o = 8 * tid;
-  uint2 v = make_uint2(0u, 0u);
-  if (!raw && o < vlen) v = ld8_nt(rec + kDenseBytes + o);
-  load_thread(rec, raw, tid, b);
-  if (raw) {
-    raw_words(b, rec, tid, emit);
+  // (a raw record has its loads to itself: with the forms' loads branched over
+  // one by one, the wait where the paths joined put a coded record's symbols a
+  // memory trip behind its low bytes)
+  if (vlen > kVarCap) {
+    raw_words(rec, tid, emit);
     return;
   }
+  SlabBuf b;
+  // the thread's 8 bytes of the variable region go out with its dense loads
+  // (past the region's end: the record's first bytes, taken as zeros)
+  const int o = 8 * tid;
+  uint2 v = ld8_nt(rec + (o < vlen ? kDenseBytes + o : 0));
+  load_thread(rec, tid, b);
+  v = o < vlen ? v : make_uint2(0u, 0u);
   // escape nibbles -> table bytes, each thread from its piece; then raw-list
   // entries patch theirs
   if (o < kHeaderBytes) {
@@ -1550,21 +1555,24 @@ __device__ void decode_record_to_tile(const uint8_t* rec, int vlen, int kv, cons
     const uint2 e0 = expand_nibbles(v.x, lut.s), e1 = expand_nibbles(v.y, lut.s);
     *reinterpret_cast<uint4*>(sh.esc + 2 * (o - kHeaderBytes)) = make_uint4(e0.x, e0.y, e1.x, e1.y);
   }
+  const int cnt = thread_escapes(b);
+  const int before = wave_incl_scan(cnt) - cnt;  // escapes before the thread, in the wave's slab
   lds_barrier();
   const int n_raw = (int)sh.hdr[1], raw_offset = (int)sh.hdr[2];
+  const int first = (int)(sh.hdr[4 + wave] & 0xFFFFu);  // escapes before the slab
+  if (n_raw > 0) {
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int off = o + 4 * q;
-    if (off >= raw_offset && ((off - raw_offset) >> 2) < n_raw) {
-      const uint32_t e = q ? v.y : v.x;
-      const int x = (int)(e & 0xFFFFu);
-      if (x < kEscLds) sh.esc[x] = (uint8_t)(e >> 16);
+    for (int q = 0; q < 2; ++q) {
+      const int off = o + 4 * q;
+      if (off >= raw_offset && ((off - raw_offset) >> 2) < n_raw) {
+        const uint32_t e = q ? v.y : v.x;
+        const int x = (int)(e & 0xFFFFu);
+        if (x < kEscLds) sh.esc[x] = (uint8_t)(e >> 16);
+      }
     }
+    lds_barrier();
   }
-  lds_barrier();
-  const int cnt = thread_escapes(b);
-  const int first = (int)(sh.hdr[4 + wave] & 0xFFFFu);  // escapes before the wave's slab
-  decode_words(b, sh.esc, first + wave_incl_scan(cnt) - cnt, lut.p0, lut.p1, emit);
+  decode_words(b, sh.esc, first + before, lut.p0, lut.p1, emit);
 }
 
 // Stores the tile: token row r to out + r * row_stride (bytes).
