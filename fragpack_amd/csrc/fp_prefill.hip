@@ -950,8 +950,10 @@ namespace {
 // - 4-wave workgroups, two per query tile (its rows by halves, ~1.3 us a key
 //   tile when a CU has one), while the 8-wave ones would leave CUs idle (1024
 //   new tokens over 2048: 76 instead of 95 us), and for fresh prompts of up to
-//   four query tiles per CU, whose tiles differ in length (2311 tokens 68 us
-//   instead of 81, 4 x 1000 59 instead of 69, 2048 x 2 89 instead of 93).  On
+//   four query tiles per CU, whose tiles differ in length under the causal mask
+//   (2311 tokens 68 us instead of 81, 4 x 1000 59 instead of 69, 2048 x 2 89
+//   instead of 93; with full attention they do not, and 2 x 2048 at H 16, G 1
+//   take 71 us with 4 waves and 68 with 8).  On
 //   full grids of equal tiles they lose, each K / V tile serving half the rows
 //   (4 x 1024 over 8192: 598 us, 8 waves 583; 4 x 8192: 2%);
 // - the split launch: ~45 us of its own (three kernels, the parts written and
@@ -979,7 +981,7 @@ struct PfLaunch {
 constexpr int64_t kPfGridMost = (1LL << 32) - 1;
 
 PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
-                        int64_t max_seqlen_k, int64_t device) {
+                        int64_t max_seqlen_k, bool causal, int64_t device) {
   const int64_t T = kPfRows / group;
   PfLaunch r;
   r.tiles = (max_seqlen_q + T - 1) / T;
@@ -987,7 +989,7 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   const int64_t most = r.tiles * num_seqs;
   const int64_t all = (total_q > 0 ? std::min(most, total_q / T + num_seqs) : most) * kv_heads;
   r.steps = all * steps;
-  const bool fresh = 2 * max_seqlen_k <= 3 * max_seqlen_q;
+  const bool fresh = causal && 2 * max_seqlen_k <= 3 * max_seqlen_q;
   r.waves = 4 * all <= 3 * cus || (fresh && all <= 4 * cus) ? 4 : kPfWaves;
   const bool split = all <= cus && 10 * (kPfSplitBase * cus + kPfSplitStep * r.steps) <
                                       kPfSplitMargin * cus * (kPfWholeBase + kPfWholeStep * steps);
@@ -1018,7 +1020,7 @@ int64_t prefill_workspace(const PfLaunch& l) {
 extern "C" int64_t fp_prefill_workspace_bytes(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
                                               int64_t max_seqlen_q, int64_t max_seqlen_k) {
   if (kv_heads < 1 || group < 1 || kPfRows % group || num_seqs < 1 || total_q < 1 || max_seqlen_q < 1) return 0;
-  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, device_cus());
+  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, true, device_cus());
   return l.split_wgs ? prefill_workspace(l) : 0;
 }
 
@@ -1034,12 +1036,12 @@ extern "C" int64_t fp_prefill_workspace_most(int64_t max_seqlen_k, int64_t cus) 
 extern "C" int64_t fp_prefill_split_min_keys(void) { return (kPfSplitSteps - 1) * kPfKeys + 1; }
 
 extern "C" int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q,
-                               int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t cus, int64_t* plan) {
+                               int64_t max_seqlen_q, int64_t max_seqlen_k, int causal, int64_t cus, int64_t* plan) {
   FP_CHECK(plan && kv_heads >= 1 && group >= 1 && kPfRows % group == 0 && num_seqs >= 1 && total_q >= 0 &&
                max_seqlen_q >= 1 && max_seqlen_k >= 0,
            "bad prefill sizes");
   const PfLaunch l =
-      prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, cus > 0 ? cus : device_cus());
+      prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, causal != 0, cus > 0 ? cus : device_cus());
   plan[0] = l.waves;
   plan[1] = l.split_wgs;
   plan[2] = l.row_wgs;
@@ -1099,7 +1101,7 @@ extern "C" int fp_prefill_attention_split(const void* q, int64_t q_stride, const
   p.causal = causal ? 1 : 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // all LDS is static (two K and two V stages, 64 KB)
-  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, device_cus());
+  const PfLaunch l = prefill_launch(kv_heads, group, num_seqs, total_q, max_seqlen_q, max_seqlen_k, causal != 0, device_cus());
   if (workspace && l.split_wgs > 0) {
     const int64_t slots = 2 * (int64_t)l.split_wgs;
     FP_CHECK(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= prefill_workspace(l),

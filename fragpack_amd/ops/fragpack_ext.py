@@ -136,7 +136,7 @@ class Extension:
             "fp_prefill_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _i64],
             "fp_prefill_workspace_most": [_i64, _i64],
             "fp_prefill_split_min_keys": [],
-            "fp_prefill_plan": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _p],
+            "fp_prefill_plan": [_i64, _i64, _i64, _i64, _i64, _i64, _i32, _i64, _p],
         }
         for name, args in sigs.items():
             fn = getattr(lib, name)

@@ -308,7 +308,7 @@ int64_t fp_prefill_split_min_keys(void);
  * as fp_prefill_attention.
  */
 int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
-                    int64_t max_seqlen_k, int64_t cus, int64_t* plan);
+                    int64_t max_seqlen_k, int causal, int64_t cus, int64_t* plan);
 
 #ifdef __cplusplus
 }

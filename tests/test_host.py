@@ -216,12 +216,12 @@ def test_plan_reuse_without_a_plan_is_refused():
         extension().fused_decode(*args, False, 0.1, G)
 
 
-def prefill_plan(heads, group, seqs, total_q, max_q, max_k, cus=256):
+def prefill_plan(heads, group, seqs, total_q, max_q, max_k, causal=True, cus=256):
     """(waves, split workgroups, workgroups of a row, rows) of a prefill call on ``cus`` compute units."""
     lib = ctypes.CDLL(str(LIB_PATH))
-    lib.fp_prefill_plan.argtypes = [ctypes.c_int64] * 7 + [ctypes.c_void_p]
+    lib.fp_prefill_plan.argtypes = [ctypes.c_int64] * 6 + [ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
     plan = (ctypes.c_int64 * 4)()
-    assert lib.fp_prefill_plan(heads, group, seqs, total_q, max_q, max_k, cus, plan) == 0
+    assert lib.fp_prefill_plan(heads, group, seqs, total_q, max_q, max_k, int(causal), cus, plan) == 0
     return tuple(plan)
 
 
@@ -274,3 +274,12 @@ def test_one_workspace_serves_every_split_call():
             tiles = min(seqs * -(-max_q // rows), total // rows + seqs) * heads
             need = 256 * (2 * 133120 + 32) + tiles * -(-max_k // 64) * 1032
             assert need <= lib.fp_prefill_workspace_most(max_k, 256)
+
+
+@pytest.mark.parametrize("heads,group,q_lens,k_lens,causal,waves", [
+    (16, 1, [2048, 2048], [2048, 2048], True, 4),  # fresh prompts: tiles of unequal length
+    (16, 1, [2048, 2048], [2048, 2048], False, 8),  # full attention: all equal, 256 of them
+    (8, 4, [1024], [1024], False, 4),  # few tiles: 8 waves would leave CUs idle
+])
+def test_prefill_waves(heads, group, q_lens, k_lens, causal, waves):
+    assert prefill_plan(heads, group, len(q_lens), sum(q_lens), max(q_lens), max(k_lens), causal)[0] == waves
