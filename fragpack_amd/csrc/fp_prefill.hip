@@ -949,7 +949,10 @@ namespace {
 //   key tiles takes ~1.7 us;
 // - 4-wave workgroups, two per query tile (its rows by halves, ~1.3 us a key
 //   tile when a CU has one), while the 8-wave ones would leave CUs idle (1024
-//   new tokens over 2048: 76 instead of 95 us), and for fresh prompts of up to
+//   new tokens over 2048: 76 instead of 95 us; but from half a CU's worth on not
+//   for sequences of one query tile over several rows of heads, whose K / V no
+//   other tile shares: 8 x 128 over 1000 at H 20, G 1 take 43.6 us with 4 waves,
+//   39 with 8, 32 x 64 over 500 at H 5 29.6 and 27.0), and for fresh prompts of up to
 //   four query tiles per CU, whose tiles differ in length under the causal mask
 //   (2311 tokens 68 us instead of 81, 4 x 1000 59 instead of 69, 2048 x 2 89
 //   instead of 93; with full attention they do not, and 2 x 2048 at H 16, G 1
@@ -980,6 +983,13 @@ struct PfLaunch {
 // work items of a grid's x dimension (HIP's limit)
 constexpr int64_t kPfGridMost = (1LL << 32) - 1;
 
+// The largest of 8, 4, 2, 1 that divides the heads.
+int head_sets(int64_t kv_heads) {
+  int sets = kPfXcds;
+  while (kv_heads % sets) sets /= 2;
+  return sets;
+}
+
 PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
                         int64_t max_seqlen_k, bool causal, int64_t device) {
   const int64_t T = kPfRows / group;
@@ -990,18 +1000,21 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   const int64_t all = (total_q > 0 ? std::min(most, total_q / T + num_seqs) : most) * kv_heads;
   r.steps = all * steps;
   const bool fresh = causal && 2 * max_seqlen_k <= 3 * max_seqlen_q;
-  r.waves = 4 * all <= 3 * cus || (fresh && all <= 4 * cus) ? 4 : kPfWaves;
+  const int sets = head_sets(kv_heads);
+  r.waves = 2 * all <= cus || (4 * all <= 3 * cus && (r.tiles > 1 || kv_heads == sets)) || (fresh && all <= 4 * cus)
+                ? 4
+                : kPfWaves;
   const bool split = all <= cus && 10 * (kPfSplitBase * cus + kPfSplitStep * r.steps) <
                                       kPfSplitMargin * cus * (kPfWholeBase + kPfWholeStep * steps);
   r.split_wgs = total_q > 0 && split && r.steps <= kPfSplitMost ? (int)cus : 0;
   // The most head sets that divide the heads and that the grid's x dimension
   // holds: a row has the query tiles of head_sets heads.
   const int64_t items = most * (kPfWaves / r.waves);
-  for (r.head_sets = kPfXcds;; r.head_sets /= 2) {
+  for (r.head_sets = sets;; r.head_sets /= 2) {
     const int64_t share = kPfXcds / r.head_sets;
     r.rows = kv_heads / r.head_sets;
     r.row_wgs = kPfXcds * ((items + share - 1) / share);
-    if (r.head_sets == 1 || (kv_heads % r.head_sets == 0 && r.row_wgs * 64 * r.waves <= kPfGridMost)) break;
+    if (r.head_sets == 1 || r.row_wgs * 64 * r.waves <= kPfGridMost) break;
   }
   // (with one head a row need not fill its last round over the XCDs)
   if (r.row_wgs * 64 * r.waves > kPfGridMost) r.row_wgs = items;
