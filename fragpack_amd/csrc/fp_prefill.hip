@@ -949,14 +949,15 @@ namespace {
 //   key tiles takes ~1.7 us;
 // - 4-wave workgroups, two per query tile (its rows by halves, ~1.3 us a key
 //   tile when a CU has one), while the 8-wave ones would leave CUs idle (1024
-//   new tokens over 2048: 76 instead of 95 us; but from half a CU's worth on not
-//   for sequences of one query tile over several rows of heads, whose K / V no
-//   other tile shares: 8 x 128 over 1000 at H 20, G 1 take 43.6 us with 4 waves,
-//   39 with 8, 32 x 64 over 500 at H 5 29.6 and 27.0), and for fresh prompts of up to
-//   four query tiles per CU, whose tiles differ in length under the causal mask
-//   (2311 tokens 68 us instead of 81, 4 x 1000 59 instead of 69, 2048 x 2 89
-//   instead of 93; with full attention they do not, and 2 x 2048 at H 16, G 1
-//   take 71 us with 4 waves and 68 with 8).  On
+//   new tokens over 2048: 76 instead of 95 us; but from half the CUs on not for
+//   sequences of one or two query tiles over several rows of heads, whose K / V
+//   few other tiles share: 8 x 128 over 1000 at H 20, G 1 take 43.6 us with 4
+//   waves, 39 with 8, 32 x 64 over 500 at H 5 29.6 and 27.0), and for fresh
+//   prompts of up to four query tiles per CU, whose tiles differ in length
+//   under the causal mask (2311 tokens 68 us instead of 81, 4 x 1000 59 instead
+//   of 69, 2048 x 2 89 instead of 93; with full attention they do not, and 4
+//   waves help only past a round: 2 x 2048 at H 16, G 1, 256 tiles, take 71 us
+//   with 4 waves and 68 with 8, at H 5, G 4, 320 tiles, 107 and 127).  On
 //   full grids of equal tiles they lose, each K / V tile serving half the rows
 //   (4 x 1024 over 8192: 598 us, 8 waves 583; 4 x 8192: 2%);
 // - the split launch: ~45 us of its own (three kernels, the parts written and
@@ -999,9 +1000,9 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   const int64_t most = r.tiles * num_seqs;
   const int64_t all = (total_q > 0 ? std::min(most, total_q / T + num_seqs) : most) * kv_heads;
   r.steps = all * steps;
-  const bool fresh = causal && 2 * max_seqlen_k <= 3 * max_seqlen_q;
+  const bool fresh = (causal || all > cus) && 2 * max_seqlen_k <= 3 * max_seqlen_q;
   const int sets = head_sets(kv_heads);
-  r.waves = 2 * all <= cus || (4 * all <= 3 * cus && (r.tiles > 1 || kv_heads == sets)) || (fresh && all <= 4 * cus)
+  r.waves = 2 * all <= cus || (4 * all <= 3 * cus && (r.tiles > 2 || kv_heads == sets)) || (fresh && all <= 4 * cus)
                 ? 4
                 : kPfWaves;
   const bool split = all <= cus && 10 * (kPfSplitBase * cus + kPfSplitStep * r.steps) <

@@ -279,12 +279,14 @@ def test_one_workspace_serves_every_split_call():
 @pytest.mark.parametrize("heads,group,q_lens,k_lens,causal,waves", [
     (16, 1, [2048, 2048], [2048, 2048], True, 4),  # fresh prompts: tiles of unequal length
     (16, 1, [2048, 2048], [2048, 2048], False, 8),  # full attention: all equal, 256 of them
+    (5, 4, [2048] * 2, [2048] * 2, False, 4),  # 320: more than a round
     (8, 4, [1024], [1024], False, 4),  # few tiles: 8 waves would leave CUs idle
     (20, 1, [128] * 8, [1128] * 8, True, 8),  # 160 tiles, one a sequence, several rows of heads
     (5, 4, [64] * 32, [564] * 32, True, 8),
     (5, 4, [64] * 24, [564] * 24, True, 4),  # 120: CUs would idle
     (8, 4, [64] * 20, [564] * 20, True, 4),  # 160, one row
-    (20, 1, [512] * 4, [1512] * 4, True, 4),  # 160, two a sequence
+    (10, 4, [128] * 8, [1128] * 8, True, 8),  # 160, two a sequence
+    (20, 1, [1024] * 2, [4096] * 2, True, 4),  # 160, four a sequence
 ])
 def test_prefill_waves(heads, group, q_lens, k_lens, causal, waves):
     assert prefill_plan(heads, group, len(q_lens), sum(q_lens), max(q_lens), max(k_lens), causal)[0] == waves
