@@ -76,7 +76,8 @@ struct PrefillParams {
   int64_t bt_stride;
   int64_t num_pages;
   int kvh, group, num_seqs, tiles_per_seq;
-  int head_sets;  // largest of 8, 4, 2, 1 that divides kvh
+  int head_sets;  // heads of a grid row: 8, 4, 2 or 1
+  int tile_major;
   float scale_log2;
   int causal;
   // split launches: parts' O, m and l, two slots per workgroup; and per key
@@ -395,9 +396,19 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     constexpr int kShares = kPfWaves / kWaves;  // workgroups per query tile
     const int t = item / kShares;
     row0 = item % kShares * (kWaves * kPfWaveRows);
-    at.b = t / p.tiles_per_seq;
-    at.tile = p.tiles_per_seq - 1 - t % p.tiles_per_seq;
-    if (at.b >= p.num_seqs) return;
+    // Where XCDs share a head, that order gives each XCD every share-th tile,
+    // the first ones the longest of every group: sequences of equal length take
+    // turns instead (tile_major), which spreads each tile index over the XCDs
+    // (prefill_launch has the rule).
+    if (p.tile_major) {
+      at.b = t % p.num_seqs;
+      at.tile = p.tiles_per_seq - 1 - t / p.num_seqs;
+      if (at.tile < 0) return;
+    } else {
+      at.b = t / p.tiles_per_seq;
+      at.tile = p.tiles_per_seq - 1 - t % p.tiles_per_seq;
+      if (at.b >= p.num_seqs) return;
+    }
   }
   for (;;) {
   const int h = at.h, b = at.b, qtile = at.tile;
@@ -980,6 +991,7 @@ struct PfLaunch {
   // the launch that does not split: heads of a grid row, rows, workgroups of a row
   int head_sets;
   int64_t rows, row_wgs;
+  bool tile_major;  // a row's order: sequences take turns
 };
 // work items of a grid's x dimension (HIP's limit)
 constexpr int64_t kPfGridMost = (1LL << 32) - 1;
@@ -1019,6 +1031,14 @@ PfLaunch prefill_launch(int64_t kv_heads, int64_t group, int64_t num_seqs, int64
   }
   // (with one head a row need not fill its last round over the XCDs)
   if (r.row_wgs * 64 * r.waves > kPfGridMost) r.row_wgs = items;
+  // Sequences of equal query length take turns where XCDs share a head and CUs
+  // get more than one workgroup of unequal tiles, or more than a round (4 x
+  // 2048 at H 5, G 4: 114 us, 140 sequence by sequence; 4 x 8192 1306, 1512; 4 x
+  // 1024 over 8192 at H 3, G 8 482, 502; 8 x 512 at H 4, G 8 37, 44).  Lengths
+  // that differ leave dead tiles at a sequence's end, which would load the XCDs
+  // unevenly (4000, 100 and 2000 at H 6, G 4: 215 us, 160).
+  r.tile_major = causal && num_seqs > 1 && sets < kPfXcds && total_q == num_seqs * max_seqlen_q &&
+                 r.rows * r.row_wgs * (fresh ? kPfWaves : r.waves) > kPfWaves * cus;
   return r;
 }
 
@@ -1060,6 +1080,7 @@ extern "C" int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs
   plan[1] = l.split_wgs;
   plan[2] = l.row_wgs;
   plan[3] = l.rows;
+  plan[4] = l.tile_major;
   return 0;
 }
 
@@ -1136,6 +1157,7 @@ extern "C" int fp_prefill_attention_split(const void* q, int64_t q_stride, const
   } else {
     FP_CHECK(l.row_wgs * 64 * l.waves <= kPfGridMost, "grid too large");
     p.head_sets = l.head_sets;
+    p.tile_major = l.tile_major;
     const dim3 grid((unsigned)l.row_wgs, (unsigned)l.rows), block(64 * l.waves);
     if (l.waves == 4)
       hipLaunchKernelGGL((prefill_kernel<4, false>), grid, block, 0, s, p);

@@ -304,8 +304,8 @@ int64_t fp_prefill_split_min_keys(void);
  * What a call of these sizes launches on a device of ``cus`` compute units (0:
  * the current one), without launching it: plan[0] waves per workgroup, plan[1]
  * workgroups of the split launch that a workspace allows (0: none), plan[2]
- * and plan[3] workgroups of a row and rows of the grid otherwise.  total_q 0:
- * as fp_prefill_attention.
+ * and plan[3] workgroups of a row and rows of the grid otherwise, plan[4] 1 if
+ * its sequences take turns.  total_q 0: as fp_prefill_attention.
  */
 int fp_prefill_plan(int64_t kv_heads, int64_t group, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
                     int64_t max_seqlen_k, int causal, int64_t cus, int64_t* plan);

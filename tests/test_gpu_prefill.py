@@ -121,6 +121,17 @@ def test_workgroup_mapping(heads, q_lens):
     _run(50 + heads, heads=heads, group=2, q_lens=q_lens, k_lens=[n + 40 * (i % 2) for i, n in enumerate(q_lens)])
 
 
+@pytest.mark.parametrize("heads,group,q_lens,k_lens", [
+    (1, 8, [70] * 5, [70] * 5),
+    (3, 2, [257] * 3, [257] * 3),
+    (4, 4, [130] * 2, [130, 190]),
+    (6, 1, [513] * 4, [513, 600, 513, 520]),
+])
+def test_equal_sequences_take_turns(heads, group, q_lens, k_lens):
+    # the grid's order where XCDs share a head (tile counts no multiple of the share)
+    _run(90 + heads, heads=heads, group=group, q_lens=q_lens, k_lens=k_lens)
+
+
 def test_a_grid_past_one_row_of_every_head():
     # 4 sequences bounded by 2^23 queries: 2^20 tiles a head, nearly all dead;
     # all 8 heads in one grid row would pass the 2^32 work items a launch takes

@@ -217,10 +217,10 @@ def test_plan_reuse_without_a_plan_is_refused():
 
 
 def prefill_plan(heads, group, seqs, total_q, max_q, max_k, causal=True, cus=256):
-    """(waves, split workgroups, workgroups of a row, rows) of a prefill call on ``cus`` compute units."""
+    """(waves, split workgroups, workgroups of a row, rows, tile-major) of a prefill call on ``cus`` compute units."""
     lib = ctypes.CDLL(str(LIB_PATH))
     lib.fp_prefill_plan.argtypes = [ctypes.c_int64] * 6 + [ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
-    plan = (ctypes.c_int64 * 4)()
+    plan = (ctypes.c_int64 * 5)()
     assert lib.fp_prefill_plan(heads, group, seqs, total_q, max_q, max_k, int(causal), cus, plan) == 0
     return tuple(plan)
 
@@ -231,7 +231,7 @@ def test_prefill_grid_covers_the_tiles_within_the_launch_limit(heads, seqs, tile
     """HIP takes fewer than 2^32 work items along x: one head's tiles fit up to
     2^23 - 1 workgroups of 512, so that many are never refused, and the rows
     hold every (query tile, head)."""
-    waves, _, row, rows = prefill_plan(heads, 8, seqs, 0, 32 * tiles, 4096)
+    waves, _, row, rows, _ = prefill_plan(heads, 8, seqs, 0, 32 * tiles, 4096)
     assert row * 64 * waves < 1 << 32
     assert rows <= heads and heads % rows == 0
     per_head = seqs * tiles * (8 // waves)
@@ -290,3 +290,16 @@ def test_one_workspace_serves_every_split_call():
 ])
 def test_prefill_waves(heads, group, q_lens, k_lens, causal, waves):
     assert prefill_plan(heads, group, len(q_lens), sum(q_lens), max(q_lens), max(k_lens), causal)[0] == waves
+
+
+@pytest.mark.parametrize("heads,q_lens,k_lens,turns", [
+    (5, [2048] * 4, [2048] * 4, True),
+    (5, [2048, 2048, 2048, 2000], [2048] * 4, False),  # lengths differ
+    (5, [2048], [2048], False),
+    (8, [2048] * 4, [2048] * 4, False),  # a head per XCD
+    (3, [1024] * 4, [9216] * 4, False),  # one round
+    (3, [4096] * 4, [12288] * 4, True),
+    (4, [512] * 4, [512] * 4, False),  # a workgroup per CU
+])
+def test_prefill_sequences_take_turns(heads, q_lens, k_lens, turns):
+    assert prefill_plan(heads, 4, len(q_lens), sum(q_lens), max(q_lens), max(k_lens))[4] == turns
