@@ -12,6 +12,8 @@ sequence.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -169,6 +171,20 @@ SPLITS = [
 
 @pytest.mark.parametrize("heads,group,q_lens,k_lens,causal", SPLITS)
 def test_split_matches_unsplit(heads, group, q_lens, k_lens, causal):
+    _split_and_unsplit(heads, group, q_lens, k_lens, causal, reference=max(k_lens) > 64)
+
+
+@pytest.mark.parametrize("heads,group,q_lens,k_lens", [
+    (1, 8, [1024], [34000]),  # ranges of more than 64 key tiles (flags kept 64 a time)
+    (1, 1, [1 + i % 3 for i in range(70)], [1600 - 9 * i for i in range(70)]),  # more than 64 sequences
+    (1, 8, [2112], [6000]),  # more than 64 query tiles of a sequence
+])
+def test_split_over_more_than_a_wave_of_everything(heads, group, q_lens, k_lens):
+    # (the unsplit launch is the reference: checked against fp32 above)
+    _split_and_unsplit(heads, group, q_lens, k_lens, True, reference=False)
+
+
+def _split_and_unsplit(heads, group, q_lens, k_lens, causal, reference):
     import torch
 
     from fragpack_amd.ops.fragpack_ext import extension
@@ -206,7 +222,7 @@ def test_split_matches_unsplit(heads, group, q_lens, k_lens, causal):
         outs.append(out.float())
     assert torch.isfinite(outs[0]).all()
     torch.testing.assert_close(outs[1], outs[0], atol=1e-4, rtol=2 ** -7)
-    if max(k_lens) > 64:
+    if reference:
         ref = _reference(q.cpu(), wk.cpu(), wv.cpu(), bt.cpu().numpy(), cu.cpu().numpy(), kl.cpu().numpy(), group,
                          D ** -0.5, causal)
         torch.testing.assert_close(outs[1].cpu(), ref, atol=ATOL, rtol=RTOL)
@@ -259,24 +275,51 @@ def test_split_workspace_from_the_caller_or_none_at_all(monkeypatch):
     (2, 8, [70, 33], [70, 200]),  # shares are head ranges
 ])
 def test_four_and_eight_wave_workgroups_agree(heads, group, q_lens, k_lens):
-    # an inflated query bound makes the grid large: the 8-wave launch (dead
-    # tiles leave at once); the same rows per wave, so the same bits
+    # the same rows per wave, so the same bits
     import torch
 
+    runs = [_with_bounds(heads, group, q_lens, k_lens, waves, seed=71 + group)[0] for waves in (4, 8)]
+    assert torch.equal(*runs)
+
+
+@pytest.mark.parametrize("heads,group,q_lens,k_lens,causal", [
+    (3, 1, [300, 1, 257], [700, 1, 1025], True),
+    (2, 2, [129, 64], [129, 900], False),
+    (1, 4, [65, 0, 200], [400, 30, 200], True),
+    (5, 8, [33, 70], [97, 640], True),
+    (4, 1, [256], [300], False),
+])
+def test_eight_wave_workgroups(heads, group, q_lens, k_lens, causal):
+    got, (q, wk, wv, bt, cu, kl) = _with_bounds(heads, group, q_lens, k_lens, 8, causal)
+    ref = _reference(q, wk, wv, bt, cu, kl, group, D ** -0.5, causal)
+    assert got.isfinite().all()
+    import torch
+
+    torch.testing.assert_close(got.float().cpu(), ref, atol=ATOL, rtol=RTOL)
+
+
+def _with_bounds(heads, group, q_lens, k_lens, waves, causal=True, seed=77):
+    """The case under size bounds for which the launch runs ``waves``-wave
+    workgroups: its own, or many query tiles that are not fresh prompts'
+    (dead tiles leave at once)."""
+    import torch
+
+    from fragpack_amd.ops.fragpack_ext import extension
     from fragpack_amd.ops.prefill_attn import flash_attn_varlen_func
 
-    q, wk, wv, bt, cu, kl = _case(71 + group, heads, group, q_lens, k_lens)
-    outs = []
-    for max_q in (max(q_lens) + len(q_lens) * 256, 128 * 256):
-        print("prefill waves", heads, group, q_lens, max_q, flush=True)
-        out = torch.full_like(q, float("nan"), device="cuda")
-        # (one call over more tokens than there are: the rows bound the tiles too)
-        big = torch.zeros((max_q, heads * group, D), dtype=torch.bfloat16, device="cuda")
-        big[: q.shape[0]] = q.cuda()
-        dst = torch.empty_like(big)
-        flash_attn_varlen_func(q=big, k=wk.cuda(), v=wv.cuda(), out=dst, cu_seqlens_q=torch.from_numpy(cu).cuda(),
-                               max_seqlen_q=max_q, seqused_k=torch.from_numpy(kl).cuda(), max_seqlen_k=max(k_lens),
-                               softmax_scale=D ** -0.5, causal=True, block_table=torch.from_numpy(bt).cuda())
-        out.copy_(dst[: q.shape[0]])
-        outs.append(out)
-    assert torch.equal(outs[0], outs[1])
+    case = q, wk, wv, bt, cu, kl = _case(seed, heads, group, q_lens, k_lens)
+    rows = max(q.shape[0], max(q_lens)) if waves == 4 else 300 * 256
+    max_q, max_k = (max(q_lens), max(k_lens)) if waves == 4 else (rows, 2 * rows)
+    plan = (ctypes.c_int64 * 5)()
+    assert extension()._lib.fp_prefill_plan(heads, group, len(q_lens), rows, max_q, max_k, int(causal), 0, plan) == 0
+    assert plan[0] == waves and plan[1] == 0, list(plan)
+    print("prefill waves", heads, group, q_lens, waves, flush=True)
+    table = np.zeros((bt.shape[0], max(bt.shape[1], -(-max_k // T))), np.int32)
+    table[:, : bt.shape[1]] = bt
+    big = torch.zeros((rows, heads * group, D), dtype=torch.bfloat16, device="cuda")
+    big[: q.shape[0]] = q.cuda()
+    out = torch.full_like(big, float("nan"))
+    flash_attn_varlen_func(q=big, k=wk.cuda(), v=wv.cuda(), out=out, cu_seqlens_q=torch.from_numpy(cu).cuda(),
+                           max_seqlen_q=max_q, seqused_k=torch.from_numpy(kl).cuda(), max_seqlen_k=max_k,
+                           softmax_scale=D ** -0.5, causal=causal, block_table=torch.from_numpy(table).cuda())
+    return out[: q.shape[0]], case
