@@ -15,9 +15,10 @@
 //   The 256 rows are T = 256 / G tokens x G query heads of the KV head
 //   (head-major), so every K / V tile read serves the whole GQA group and
 //   eight waves.  Wave w owns rows 32w .. 32w + 31 as two 16-column MFMA
-//   tiles.  Grids of no more tiles than CUs run two 4-wave workgroups per tile,
-//   and still smaller ones with long contexts split the keys over the CUs
-//   (below; prefill_launch has the rules).
+//   tiles.  Grids that would leave CUs idle, and fresh prompts of few tiles a
+//   CU, run two 4-wave workgroups per tile; grids of no more tiles than CUs
+//   over long contexts split the keys over the CUs (below; prefill_launch has
+//   the rules).
 // * Keys stream in 64-key tiles through double-buffered LDS, K and V both
 //   key-major and loaded straight from HBM into LDS (buffer_load ... lds, no
 //   registers).  K fragments are plain 16-byte reads; V^T fragments come
@@ -389,7 +390,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     // Tiles of one sequence thus spread over all XCDs and CUs: with the
     // sequence as the fastest index a long one among short ones ran on a
     // quarter of the device (prompts of 1000, 37, 2311 and 512 tokens at H 8,
-    // G 4: 218 us, now 81 us).
+    // G 4: 218 us, 81 in this order, 74 with 4-wave workgroups).
     const int xcd = (int)blockIdx.x % kPfXcds, share = kPfXcds / p.head_sets;
     const int item = (int)blockIdx.x / kPfXcds * share + xcd / p.head_sets;
     at.h = xcd % p.head_sets + p.head_sets * (int)blockIdx.y;
@@ -523,7 +524,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   // next tile's loads right after issuing them.
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   // V fragment lanes: row x = 4 q4 + j / 4 of each 16-row block, byte
-  // 8 (j & 1) of the chunk; the chunk's slot term 16 ((j >> 1 & 1) ^ x)
+  // 8 (j & 1) of the chunk; the chunk's slot term 16 ((j >> 1 & 1) ^ 2 (x % 8))
   const int vx = 4 * q4 + (j >> 2);
   const int vlane = vx * kKRow + 8 * (j & 1), vsw = 16 * (((j >> 1) & 1) ^ tile_swizzle<true>(vx));
   auto tile = [&](int it, const uint8_t* stage, uint8_t* knext, const uint8_t* vstage, uint8_t* vnext)
@@ -675,7 +676,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
         // chunk 2 dt + (j >> 1 & 1) of row x = 4 q4 + j / 4 (mod 16) sits at
-        // slot chunk ^ x
+        // slot chunk ^ 2 (x % 8)
         const uint8_t* base = vstage + (vsw ^ (32 * dt)) + vlane;
         const uint2 lo = lds_tr16(base + 32 * kk * kKRow);
         const uint2 hi = lds_tr16(base + (32 * kk + 16) * kKRow);
@@ -741,10 +742,11 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 // Column maxima for the parts' references (see above): every range but the
 // parts that end their query tile, which none follows.  Grid as the split
 // prefill's.  Bound by its steps' latency (K fragments from LDS, one barrier a
-// key tile: ~1.1 us, 1.4 with every tile masked and its columns reduced), 25
-// us of the 76 that 200 tokens over 8192 take (H 4, G 8; 9 parts a tile); the
-// parts take 54 (14 of launch and first loads, ~7 of replays, 4 of stores,
-// ~1.9 a key tile) and the merge 10.
+// key tile: ~1.1 us, 1.4 with every tile masked and its columns reduced).  200
+// tokens over 8192 (H 4, G 8; 9 parts a tile) take 73-77 us in a timed loop; in
+// a kernel trace, which adds to each launch, this kernel shows 25, the parts 54
+// (14 of launch and first loads, ~7 of replays, 4 of stores, ~1.9 a key tile)
+// and the merge 10.
 __global__ void __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(kPfWavesPerEu))) prefill_max_kernel(PrefillParams p) {
   // four stages: a step is shorter than a memory round trip, so transfers run
   // three key tiles ahead

@@ -47,7 +47,9 @@ def flash_attn_varlen_func(
         cu_seqlens_q: int32 ``[B + 1]`` query offsets.
         max_seqlen_q: Largest query count (sizes the launch grid).
         seqused_k: int32 ``[B]`` key counts.
-        max_seqlen_k: Largest key count.
+        max_seqlen_k: Largest key count; it also chooses the launch, and a
+            bound far above the real one costs a short call the split
+            launch's three kernels (16 tokens: 28 us, 6 with their own).
         softmax_scale: Defaults to ``128 ** -0.5``.
         causal: Bottom-right aligned causal mask.
         block_table: int32 ``[B, pages]`` workspace pages per sequence.
@@ -63,7 +65,10 @@ def flash_attn_varlen_func(
         Enqueues on the current stream; not synchronized.
 
     A call with few query tiles over long contexts splits its keys over the
-    GPU and takes up to ~140 MB for the parts from torch's allocator for its
+    GPU: the parts are cut by the whole call's key tiles, so a row's sums may
+    add up in another order beside other sequences than alone (its output then
+    differs by at most one BF16 step; the same call gives the same bits).  It
+    takes up to ~140 MB for the parts from torch's allocator for its
     duration (without that much free it runs unsplit); a caller with a
     workspace of its own uses :func:`prefill_attention`.
     """

@@ -278,8 +278,11 @@ int fp_prefill_attention(const void* q, int64_t q_stride, const void* wk, const 
 /*
  * fp_prefill_attention with a workspace, which lets the launch split the keys
  * of long query tiles over the device's CUs and merge the parts: few query
- * tiles, or tiles of unequal length, then still fill the chip.  total_q (the
- * rows of q) bounds the query tiles.  workspace: device memory of
+ * tiles, or tiles of unequal length, then still fill the chip.  The parts are
+ * cut by the whole call's key tiles: a row's fp32 sums may add up in another
+ * order beside other sequences than alone (at most one BF16 step).  total_q (the
+ * rows of q) bounds the query tiles, and max_seqlen_k the key tiles: a bound far
+ * above the real one splits short calls.  workspace: device memory of
  * fp_prefill_workspace_bytes for the same sizes, 16-byte aligned, contents
  * irrelevant before and after; calls that may overlap need one each.  A null
  * workspace (or 0 bytes asked for) runs fp_prefill_attention's launch.
