@@ -305,11 +305,17 @@ class FragPackRunner:
         self.wk = torch.empty(shape, dtype=torch.bfloat16, device=self.device)
         self.wv = torch.empty(shape, dtype=torch.bfloat16, device=self.device)
         # parts of the prefill calls that split their keys over the CUs (any
-        # call of up to max_model_len keys): a full device then refuses the
-        # runner, not a prefill in mid-serving
+        # call of up to max_model_len keys), held from the start so that no
+        # prefill needs memory in mid-serving; a device too full for it runs
+        # those calls unsplit
         with torch.cuda.device(self.device):
             split_bytes = extension().prefill_workspace_bytes(max_model_len)
-        self.split_workspace = torch.empty(split_bytes, dtype=torch.uint8, device=self.device)
+        try:
+            self.split_workspace = torch.empty(split_bytes, dtype=torch.uint8, device=self.device)
+        except torch.OutOfMemoryError:
+            logger.warning("FragPack: no room for the %.0f MiB split-prefill workspace; short prefills over long "
+                           "contexts run unsplit", split_bytes / 2**20)
+            self.split_workspace = torch.empty(0, dtype=torch.uint8, device=self.device)
         self.store = None
         self.store_key: tuple[int, int] | None = None
         self.layer_tables: list = []

@@ -248,9 +248,11 @@ def test_engine_steps_match_fp32_attention(driver, monkeypatch, tmp_path):
     assert cap.memory["arena"] == NB * L * cap.page_bytes
 
 
-def test_a_layer_allocates_nothing(monkeypatch):
+@pytest.mark.parametrize("full", [False, True])
+def test_a_layer_allocates_nothing(full, monkeypatch):
     """A step's layers run in what the runner holds and publishes: a short
-    chunk over a long context (the split prefill) allocates no device memory."""
+    chunk over a long context (the split prefill) allocates no device memory.
+    ``full``: a device without room for the split workspace still serves."""
     import torch
 
     from fragpack_amd.compression.attn_tables import device_tables
@@ -263,6 +265,16 @@ def test_a_layer_allocates_nothing(monkeypatch):
     rng = np.random.default_rng(63)
     tables = workloads.calibrated_tables(rng, H, workloads.channel_scales(rng, H, 0.02))
     caches = [torch.empty((pages, page_bytes(H)), dtype=torch.uint8, device="cuda")]
+    most, empty = extension().prefill_workspace_bytes(ctx + chunk), torch.empty
+    need = extension()._lib.fp_prefill_workspace_bytes(H, G, 1, chunk, chunk, ctx + chunk)
+
+    def no_room(*size, **kw):
+        if size in ((most,), (need,)):
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    if full:
+        monkeypatch.setattr(torch, "empty", no_room)
     runner = FragPackRunner(H, device_tables(tables, torch.device("cuda")), "cuda", ctx, 1, ctx + chunk, 64)
     table = torch.arange(pages, dtype=torch.int32, device="cuda")[None]
     gen = torch.Generator(device="cuda").manual_seed(64)
@@ -279,6 +291,6 @@ def test_a_layer_allocates_nothing(monkeypatch):
         layer_forward(md, 0, q, kv[0], kv[1], out, D ** -0.5)
         assert torch.cuda.memory_stats()["allocation.all.allocated"] == before, n
         done += n
-    assert extension()._lib.fp_prefill_workspace_bytes(H, G, 1, chunk, chunk, ctx + chunk) > 0
+    assert most >= need > 0
     assert torch.isfinite(out).all()
-    assert get_capacity().memory["prefill_split_workspace"] == extension().prefill_workspace_bytes(ctx + chunk) > 0
+    assert get_capacity().memory["prefill_split_workspace"] == (0 if full else most)
