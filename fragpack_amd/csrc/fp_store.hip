@@ -609,77 +609,69 @@ __global__ void __launch_bounds__(kPrepThreads) prepare_kernel(Store s, const in
   }
   // One pass over the slot mapping: two lists compacted together in input order
   // -- the block of every offset-0 token and of every offset-127 token (with
-  // its close mark) -- into LDS (kFits: until a round passes kPrepThreads
-  // entries), and past that into prepare_many's.  Counts are packed in one
-  // scan (each below 2^16: kScanPer * kPrepThreads items per round); the next
-  // round's slots load while a round is scanned (the barriers wait for LDS
-  // only).  Two loops, so that the common one holds no pointers of the other
-  // (8192 tokens a round, 16 rounds: 58.7 us in one loop, 54.7 in two).
-  // Returns the round it stopped at.
+  // its close mark) -- into LDS until a round passes kPrepThreads entries, and
+  // from there into prepare_many's.  Counts are packed in one scan (each below
+  // 2^16: kScanPer * kPrepThreads items per round); the next round's slots load
+  // while a round is scanned (the barriers wait for LDS only).  Two loops, so
+  // that the common one holds no pointers of the other (8192 tokens a round, 16
+  // rounds: 58.7 us in one loop, 56 in two).
   StepTokenCounts n{0, 0};
-  auto scan = [&](auto fits_c, int r0) __attribute__((always_inline)) {
-    constexpr bool kFits = decltype(fits_c)::value;
-    for (; r0 < n_tok; r0 += kScanPer * kPrepThreads) {
-      int b0[kScanPer], b1[kScanPer], c = 0;
-#pragma unroll
-      for (int k = 0; k < kScanPer; ++k) {
-        b0[k] = slot_block(s, nv[k], 0);
-        b1[k] = slot_block(s, nv[k], 127);
-        c += (b0[k] >= 0) + ((b1[k] >= 0) << 16);
-      }
-      const int i1 = r0 + kScanPer * (kPrepThreads + tid);
-#pragma unroll
-      for (int k = 0; k < kScanPer; ++k) nv[k] = i1 + k < n_tok ? slots[i1 + k] : -1;
-      int all = 0;
-      const int ex = wg_prefix(c, sh, all);
-      int r0c = n.raw0 + (ex & 0xFFFF), r1c = n.raw1 + (ex >> 16);
-      if constexpr (kFits) {
-        if (n.raw0 + (all & 0xFFFF) > kPrepThreads || n.raw1 + (all >> 16) > kPrepThreads) break;
-#pragma unroll
-        for (int k = 0; k < kScanPer; ++k) {
-          if (b0[k] >= 0) f.cand[r0c++] = b0[k];
-          if (b1[k] >= 0) {
-            f.ccand[r1c++] = b1[k];
-            atomicOr(&f.close_mark[(b1[k] >> 5) & (kFewWords - 1)], 1u << (b1[k] & 31));  // (read only with ``marks``)
-          }
-        }
-      } else {
-        int32_t* tmp = s.close_list;
-        int32_t* ccand = s.close_list + s.cap;
-        int32_t* close_tag = s.tags + kTagClose * s.NB;
-#pragma unroll
-        for (int k = 0; k < kScanPer; ++k) {
-          if (b0[k] >= 0) {
-            if (r0c < kPrepThreads)
-              f.cand[r0c] = b0[k];
-            else
-              tmp[r0c] = b0[k];
-            ++r0c;
-          }
-          if (b1[k] >= 0) {
-            if (r1c < kPrepThreads) {
-              f.ccand[r1c] = b1[k];
-            } else {
-              ccand[r1c] = b1[k];
-              close_tag[b1[k]] = step;
-            }
-            ++r1c;
-          }
-        }
-      }
-      n.raw0 += all & 0xFFFF;
-      n.raw1 += all >> 16;
-    }
-    return r0;
-  };
-  const int r0 = scan(std::true_type{}, 0);
-  if (r0 < n_tok) {
+  int b0[kScanPer], b1[kScanPer], r0c = 0, r1c = 0, all = 0;
+  auto scan = [&](int r0) __attribute__((always_inline)) {
+    int c = 0;
 #pragma unroll
     for (int k = 0; k < kScanPer; ++k) {
-      const int i = r0 + kScanPer * tid + k;
-      nv[k] = i < n_tok ? slots[i] : -1;
+      b0[k] = slot_block(s, nv[k], 0);
+      b1[k] = slot_block(s, nv[k], 127);
+      c += (b0[k] >= 0) + ((b1[k] >= 0) << 16);
     }
-    scan(std::false_type{}, r0);
+    const int i1 = r0 + kScanPer * (kPrepThreads + tid);
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) nv[k] = i1 + k < n_tok ? slots[i1 + k] : -1;
+    const int ex = wg_prefix(c, sh, all);
+    r0c = n.raw0 + (ex & 0xFFFF);
+    r1c = n.raw1 + (ex >> 16);
+    n.raw0 += all & 0xFFFF;
+    n.raw1 += all >> 16;
+  };
+  int r0 = 0;
+  for (; r0 < n_tok; r0 += kScanPer * kPrepThreads) {
+    scan(r0);
+    if (n.raw0 > kPrepThreads || n.raw1 > kPrepThreads) break;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+      if (b0[k] >= 0) f.cand[r0c++] = b0[k];
+      if (b1[k] >= 0) {
+        f.ccand[r1c++] = b1[k];
+        atomicOr(&f.close_mark[(b1[k] >> 5) & (kFewWords - 1)], 1u << (b1[k] & 31));  // (read only with ``marks``)
+      }
+    }
+  }
+  while (r0 < n_tok) {  // the round that did not fit, and those after it
+    int32_t* tmp = s.close_list;
+    int32_t* ccand = s.close_list + s.cap;
+    int32_t* close_tag = s.tags + kTagClose * s.NB;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+      if (b0[k] >= 0) {
+        if (r0c < kPrepThreads)
+          f.cand[r0c] = b0[k];
+        else
+          tmp[r0c] = b0[k];
+        ++r0c;
+      }
+      if (b1[k] >= 0) {
+        if (r1c < kPrepThreads) {
+          f.ccand[r1c] = b1[k];
+        } else {
+          ccand[r1c] = b1[k];
+          close_tag[b1[k]] = step;
+        }
+        ++r1c;
+      }
+    }
+    r0 += kScanPer * kPrepThreads;
+    if (r0 < n_tok) scan(r0);
   }
   lds_barrier();  // the lists and marks are in LDS
   if (__builtin_expect(marks && n.raw0 <= kPrepThreads && n.raw1 <= kPrepThreads, 1))
