@@ -462,8 +462,8 @@ def layer_forward(md: FragPackMetadata, li: int, query, key, value, output, scal
     Returns:
         ``output``.
     """
+    from fragpack_amd.ops.fragpack_ext import extension
     from fragpack_amd.ops.fused_attn_decode import decode_attention
-    from fragpack_amd.ops.prefill_attn import prefill_attention
 
     if md is None:
         return output.zero_()
@@ -483,9 +483,10 @@ def layer_forward(md: FragPackMetadata, li: int, query, key, value, output, scal
                          md.units, output[:nd], md.decode_workspace, replan=li == 0)
     for g in md.prefills:
         store.gather(li, g.src_blocks, md.wk, md.wv)
-        prefill_attention(query[g.tok0 : g.tok1], md.wk, md.wv, output[g.tok0 : g.tok1], g.cu_seqlens_q,
-                          g.max_seqlen_q, g.seqused_k, g.max_seqlen_k, scale, True, g.block_table,
-                          workspace=md.split_workspace)
+        # flash_attn_varlen_func's call, with the runner's workspace
+        extension().prefill_attention(query[g.tok0 : g.tok1], md.wk, md.wv, output[g.tok0 : g.tok1], g.cu_seqlens_q,
+                                      g.seqused_k, g.block_table, g.max_seqlen_q, g.max_seqlen_k,
+                                      HEAD_DIM ** -0.5 if scale is None else scale, True, md.split_workspace)
     if not fused:
         store.encode(li, md.max_close)
     if li == md.last_layer:

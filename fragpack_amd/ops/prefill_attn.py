@@ -70,42 +70,17 @@ def flash_attn_varlen_func(
     differs by at most one BF16 step; the same call gives the same bits).  It
     takes up to ~140 MB for the parts from torch's allocator for its
     duration (without that much free it runs unsplit); a caller with a
-    workspace of its own uses :func:`prefill_attention`.
+    workspace of its own passes it to ``extension().prefill_attention``.
     """
     del fa_version
-    return prefill_attention(q, k, v, out, cu_seqlens_q, max_seqlen_q, seqused_k, max_seqlen_k, softmax_scale, causal,
-                             block_table)
-
-
-def prefill_attention(
-    q: torch.Tensor,
-    k: torch.Tensor,
-    v: torch.Tensor,
-    out: torch.Tensor | None,
-    cu_seqlens_q: torch.Tensor | None,
-    max_seqlen_q: int,
-    seqused_k: torch.Tensor | None,
-    max_seqlen_k: int,
-    softmax_scale: float | None,
-    causal: bool,
-    block_table: torch.Tensor | None,
-    workspace: torch.Tensor | None = None,
-) -> torch.Tensor:
-    """:func:`flash_attn_varlen_func` with the caller's workspace.
-
-    Args:
-        workspace: uint8 device memory of ``extension().prefill_workspace_bytes
-            (max_seqlen_k)`` for a split call's parts, which no overlapping
-            call uses; None or too small: allocated by the call if it splits.
-    """
     if cu_seqlens_q is None or seqused_k is None or block_table is None:
         raise ValueError("cu_seqlens_q, seqused_k and block_table are required (paged varlen form)")
     if out is None:
         out = torch.empty_like(q)
     scale = softmax_scale if softmax_scale is not None else q.size(-1) ** -0.5
     extension().prefill_attention(q, k, v, out, cu_seqlens_q, seqused_k, block_table, max_seqlen_q, max_seqlen_k,
-                                  scale, causal, workspace=workspace)
+                                  scale, causal)
     return out
 
 
-__all__ = ["flash_attn_varlen_func", "prefill_attention"]
+__all__ = ["flash_attn_varlen_func"]

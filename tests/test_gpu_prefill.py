@@ -235,7 +235,7 @@ def test_split_workspace_from_the_caller_or_none_at_all(monkeypatch):
     import torch
 
     from fragpack_amd.ops.fragpack_ext import extension
-    from fragpack_amd.ops.prefill_attn import prefill_attention
+    from fragpack_amd.ops.prefill_attn import flash_attn_varlen_func
 
     ext = extension()
     q, wk, wv, bt, cu, kl = (torch.from_numpy(x).cuda() if isinstance(x, np.ndarray) else x.cuda()
@@ -243,7 +243,11 @@ def test_split_workspace_from_the_caller_or_none_at_all(monkeypatch):
     assert ext._lib.fp_prefill_workspace_bytes(2, 4, 2, 121, 120, 4000) > 0
 
     def run(out, workspace=None):
-        return prefill_attention(q, wk, wv, out, cu, 120, kl, 4000, None, True, bt, workspace=workspace)
+        if workspace is None:
+            return flash_attn_varlen_func(q=q, k=wk, v=wv, out=out, cu_seqlens_q=cu, max_seqlen_q=120, seqused_k=kl,
+                                          max_seqlen_k=4000, block_table=bt)
+        ext.prefill_attention(q, wk, wv, out, cu, kl, bt, 120, 4000, D ** -0.5, True, workspace)
+        return out
 
     want = run(torch.empty_like(q))
     ws = torch.empty(ext.prefill_workspace_bytes(4000), dtype=torch.uint8, device="cuda")
