@@ -77,8 +77,7 @@ struct PrefillParams {
   int64_t bt_stride;
   int64_t num_pages;
   int kvh, group, num_seqs, tiles_per_seq;
-  int head_sets;  // heads of a grid row: 8, 4, 2 or 1
-  int tile_major;
+  int head_sets;  // heads of a grid row: 8, 4, 2 or 1; negated: its sequences take turns
   float scale_log2;
   int causal;
   // split launches: parts' O, m and l, two slots per workgroup; and per key
@@ -391,25 +390,21 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     // sequence as the fastest index a long one among short ones ran on a
     // quarter of the device (prompts of 1000, 37, 2311 and 512 tokens at H 8,
     // G 4: 218 us, 81 in this order, 74 with 4-wave workgroups).
-    const int xcd = (int)blockIdx.x % kPfXcds, share = kPfXcds / p.head_sets;
-    const int item = (int)blockIdx.x / kPfXcds * share + xcd / p.head_sets;
-    at.h = xcd % p.head_sets + p.head_sets * (int)blockIdx.y;
+    const int sets = abs(p.head_sets), xcd = (int)blockIdx.x % kPfXcds, share = kPfXcds / sets;
+    const int item = (int)blockIdx.x / kPfXcds * share + xcd / sets;
+    at.h = xcd % sets + sets * (int)blockIdx.y;
     constexpr int kShares = kPfWaves / kWaves;  // workgroups per query tile
     const int t = item / kShares;
     row0 = item % kShares * (kWaves * kPfWaveRows);
     // Where XCDs share a head, that order gives each XCD every share-th tile,
     // the first ones the longest of every group: sequences of equal length take
-    // turns instead (tile_major), which spreads each tile index over the XCDs
+    // turns instead (head_sets < 0), which spreads each tile index over the XCDs
     // (prefill_launch has the rule).
-    if (p.tile_major) {
-      at.b = t % p.num_seqs;
-      at.tile = p.tiles_per_seq - 1 - t / p.num_seqs;
-      if (at.tile < 0) return;
-    } else {
-      at.b = t / p.tiles_per_seq;
-      at.tile = p.tiles_per_seq - 1 - t % p.tiles_per_seq;
-      if (at.b >= p.num_seqs) return;
-    }
+    const bool turns = p.head_sets < 0;
+    const int width = turns ? p.num_seqs : p.tiles_per_seq, q = t / width, m = t - q * width;
+    at.b = turns ? m : q;
+    at.tile = p.tiles_per_seq - 1 - (turns ? q : m);
+    if (at.b >= p.num_seqs || at.tile < 0) return;
   }
   for (;;) {
   const int h = at.h, b = at.b, qtile = at.tile;
@@ -1158,8 +1153,7 @@ extern "C" int fp_prefill_attention_split(const void* q, int64_t q_stride, const
                        s, p);
   } else {
     FP_CHECK(l.row_wgs * 64 * l.waves <= kPfGridMost, "grid too large");
-    p.head_sets = l.head_sets;
-    p.tile_major = l.tile_major;
+    p.head_sets = l.tile_major ? -l.head_sets : l.head_sets;
     const dim3 grid((unsigned)l.row_wgs, (unsigned)l.rows), block(64 * l.waves);
     if (l.waves == 4)
       hipLaunchKernelGGL((prefill_kernel<4, false>), grid, block, 0, s, p);
